@@ -268,7 +268,9 @@ int pbf_get_shapes(const pbf_solver* s, pbf_shapes* out);
  * the smallest of 64, 80, 96, 112, 128, 160, 192 such that the previous
  * neighbour pass found at most 1 in 25 targets with more candidates than it
  * and at most 256, else 256; otherwise a fixed count >= 64.  Like the launch
- * shapes, it changes no result, only the speed.
+ * shapes, it changes no result of a step, only the speed.  Steps of up to
+ * 90,112 particles have no chunk kernel under the adaptive setting (a team of
+ * lanes per target instead); a fixed count keeps them on the chunk kernel.
  */
 int pbf_set_heavy_threshold(pbf_solver* s, int threshold);
 int pbf_get_heavy_threshold(const pbf_solver* s, int* out);

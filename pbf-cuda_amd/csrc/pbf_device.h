@@ -172,6 +172,9 @@ typedef int pbf_i32x4 __attribute__((ext_vector_type(4)));
 typedef float pbf_f32x3 __attribute__((ext_vector_type(3)));
 __device__ pbf_f32x3 pbf_raw_buffer_load_f32x3(pbf_i32x4 rsrc, int voffset, int soffset,
                                                int aux) __asm("llvm.amdgcn.raw.buffer.load.v3f32");
+typedef float pbf_f32x4 __attribute__((ext_vector_type(4)));
+__device__ pbf_f32x4 pbf_raw_buffer_load_f32x4(pbf_i32x4 rsrc, int voffset, int soffset,
+                                               int aux) __asm("llvm.amdgcn.raw.buffer.load.v4f32");
 struct Float4Buf {
   pbf_i32x4 r;
 };
@@ -189,6 +192,12 @@ __device__ __forceinline__ Float4Buf float4_buf(const float4* p, uint32_t n) {
 __device__ __forceinline__ float3 load_xyz_at(const Float4Buf& b, uint32_t off) {
   const pbf_f32x3 v = pbf_raw_buffer_load_f32x3(b.r, (int)off, 0, 0);
   return make_float3(v.x, v.y, v.z);
+}
+
+// The element at byte offset `off`.
+__device__ __forceinline__ float4 load_f4_at(const Float4Buf& b, uint32_t off) {
+  const pbf_f32x4 v = pbf_raw_buffer_load_f32x4(b.r, (int)off, 0, 0);
+  return make_float4(v.x, v.y, v.z, v.w);
 }
 
 // Entries of a column table: nine columns and the closing entry.

@@ -24,6 +24,7 @@
 
 #include "pbf_device.h"
 #include "pbf_launch.h"
+#include "pbf_team.h"
 
 namespace pbf {
 namespace {
@@ -464,10 +465,40 @@ int grid_for_items(long long items, int max_blocks) {
   return (int)(b < 1 ? 1 : (b > max_blocks ? max_blocks : b));
 }
 
+// Lanes per target for n particles: 0 = the light, chunk and combine kernels.
+// Steps under graph replay, microseconds, fresh lattice / collapsing dam (20
+// frames) / spread dam (50 frames): 16K particles 235 / 189 / 201 with 16
+// lanes, 225 / 217 / 227 with 8, 386 / 719 / 710 with the lane kernels; 32K
+// 326 / 317 / 220, 266 / 357 / 246 and 425 / 766 / 793; 80K with 8 lanes 413 /
+// 520 / 482, 96K 495 / 542 / 601 against 469 / 836 / 935 with the lane kernels,
+// which from there on have wavefronts enough to win where every target has
+// much the same number of candidates.
+// A fixed heavy threshold asks for the chunk kernels, so it keeps the lane
+// kernels at every size.  Every choice sums in the canonical order.
+constexpr int kTeam16Max = 20480;
+constexpr int kTeam8Max = 90112;
+inline int team_lanes(int n, const Shapes& sh) {
+  if (sh.heavy != 0 || n > kTeam8Max) return 0;
+  return n <= kTeam16Max ? 16 : 8;
+}
+inline int team_blocks(int n, int lanes) {
+  const int targets = kTeamBlock / lanes;
+  return (n + targets - 1) / targets;
+}
+
 template <class P, class S>
 void launch_pass_s(const typename P::Args& a, int n, const StepConsts& c, const S& sc,
                    const uint32_t* cs, const HeavyLists& hl, int pass, const Shapes& sh,
                    hipStream_t st) {
+  const int team = team_lanes(n, sh);
+  if (team == 16) {
+    k_team<P, S, 16><<<team_blocks(n, 16), kTeamBlock, 0, st>>>(a, n, c, sc, cs);
+    return;
+  }
+  if (team == 8) {
+    k_team<P, S, 8><<<team_blocks(n, 8), kTeamBlock, 0, st>>>(a, n, c, sc, cs);
+    return;
+  }
   const int lb = sh.light_block;
   k_light<P, S><<<(n + lb - 1) / lb, lb, light_lds_bytes(lb, StageMode<P>::value), st>>>(
       a, n, c, sc, cs, hl, pass, (uint32_t)sh.heavy);

@@ -91,6 +91,32 @@ struct LambdaPass {
       }
     }
   }
+  // add() as a term and its fold (pbf_team.h); a is 0 outside the gradient's
+  // range, w outside poly6's
+  static constexpr bool kNbIsScreen = true;
+  struct Term {
+    float ax, ay, az, w;
+  };
+  static __device__ __forceinline__ Term term(const Target& t, const float4& xj,
+                                              const StepConsts& c, const Args&) {
+    float dx, dy, dz;
+    const float r2 = dist2(t.x, xj, dx, dy, dz);
+    const float r = sqrt_pair(r2);
+    const float u = c.h - r;
+    const float f = div_pair((c.spiky_rho0 * u) * u, r);
+    const bool in = (r >= c.keps) & (r < c.h);
+    return Term{in ? f * dx : 0.0f, in ? f * dy : 0.0f, in ? f * dz : 0.0f,
+                r2 < c.h2 ? poly6_of(r2, c) : 0.0f};
+  }
+  static __device__ __forceinline__ void fold(Acc& s, const Term& m) {
+    s.rho = s.rho + m.w;
+    s.gx = s.gx + m.ax;
+    s.gy = s.gy + m.ay;
+    s.gz = s.gz + m.az;
+    s.gl2 = fmaf(m.ax, m.ax, s.gl2);
+    s.gl2 = fmaf(m.ay, m.ay, s.gl2);
+    s.gl2 = fmaf(m.az, m.az, s.gl2);
+  }
   static __device__ __forceinline__ void accumulate(Acc& tot, const Acc& p) {
     tot.rho = tot.rho + p.rho;
     tot.gx = tot.gx + p.gx;
@@ -167,6 +193,30 @@ struct DeltaPass {
         s.pz = fmaf(f, dz, s.pz);
       }
     }
+  }
+  // add() as a term and its fold (pbf_team.h); i itself has r = 0 and gives
+  // a zero term
+  static constexpr bool kNbIsScreen = true;
+  struct Term {
+    float f, dx, dy, dz;
+  };
+  static __device__ __forceinline__ Term term(const Target& t, const float4& xj,
+                                              const StepConsts& c, const Args&) {
+    float dx, dy, dz;
+    const float r2 = dist2(t.x, xj, dx, dy, dz);
+    const float r = sqrt_pair(r2);
+    const float w = r2 < c.h2 ? poly6_of(r2, c) : 0.0f;
+    const float corr = c.coef_corr * pow_corr(w, c);
+    const float u = c.h - r;
+    const float gs = div_pair((c.spiky * u) * u, r);
+    const bool in = (r >= c.keps) & (r < c.h);
+    return Term{in ? ((t.x.w + xj.w) + corr) * gs : 0.0f, in ? dx : 0.0f, in ? dy : 0.0f,
+                in ? dz : 0.0f};
+  }
+  static __device__ __forceinline__ void fold(Acc& s, const Term& m) {
+    s.px = fmaf(m.f, m.dx, s.px);
+    s.py = fmaf(m.f, m.dy, s.py);
+    s.pz = fmaf(m.f, m.dz, s.pz);
   }
   static __device__ __forceinline__ void accumulate(Acc& tot, const Acc& p) {
     tot.px = tot.px + p.px;
@@ -276,6 +326,26 @@ struct XsphPass {
       s.az = fmaf(vj.z - t.v.z, f, s.az);
     }
   }
+  // add() as a term and its fold (pbf_team.h)
+  static constexpr bool kNbIsScreen = false;
+  struct Term {
+    float f, dx, dy, dz;
+  };
+  static __device__ __forceinline__ Term term(const Target& t, const Nb& nb, const StepConsts& c,
+                                              const Args&) {
+    float dx, dy, dz;
+    const float r2 = dist2(t.x, nb.x, dx, dy, dz);
+    const float w = poly6_of(r2, c);
+    const float f = div_pair(2.0f * w, t.v.w + nb.v.w);
+    const bool in = r2 < c.h2;
+    return Term{in ? f : 0.0f, in ? nb.v.x - t.v.x : 0.0f, in ? nb.v.y - t.v.y : 0.0f,
+                in ? nb.v.z - t.v.z : 0.0f};
+  }
+  static __device__ __forceinline__ void fold(Acc& s, const Term& m) {
+    s.ax = fmaf(m.dx, m.f, s.ax);
+    s.ay = fmaf(m.dy, m.f, s.ay);
+    s.az = fmaf(m.dz, m.f, s.az);
+  }
   static __device__ __forceinline__ void accumulate(Acc& tot, const Acc& p) {
     tot.ax = tot.ax + p.ax;
     tot.ay = tot.ay + p.ay;
@@ -322,6 +392,18 @@ struct DensityPass {
     const float r2 = dist2(t.x, xj, dx, dy, dz);
     if (r2 < c.h2) s.rho = s.rho + poly6_of(r2, c);
   }
+  // add() as a term and its fold (pbf_team.h)
+  static constexpr bool kNbIsScreen = true;
+  struct Term {
+    float w;
+  };
+  static __device__ __forceinline__ Term term(const Target& t, const float4& xj,
+                                              const StepConsts& c, const Args&) {
+    float dx, dy, dz;
+    const float r2 = dist2(t.x, xj, dx, dy, dz);
+    return Term{r2 < c.h2 ? poly6_of(r2, c) : 0.0f};
+  }
+  static __device__ __forceinline__ void fold(Acc& s, const Term& m) { s.rho = s.rho + m.w; }
   static __device__ __forceinline__ void accumulate(Acc& tot, const Acc& p) {
     tot.rho = tot.rho + p.rho;
   }
@@ -353,8 +435,8 @@ __global__ __launch_bounds__(kBlock) void k_predict_key(const float* __restrict_
                                                         uint32_t* __restrict__ counters) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i == 0) {
-    counters[rec_counter(0)] = 0u;
-    counters[item_counter(0)] = 0u;
+    counters[rec_counter(0)] = counters[rec_counter(1)] = 0u;
+    counters[item_counter(0)] = counters[item_counter(1)] = 0u;
   }
   if (blockIdx.x * kBlock >= n) return;  // whole workgroup past the end
   const int ii = i < n ? i : n - 1;      // idle lanes repeat the last particle
@@ -383,8 +465,8 @@ __global__ __launch_bounds__(kBlock) void k_key_only(const float* __restrict__ p
                                                      uint32_t* __restrict__ counters) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i == 0) {
-    counters[rec_counter(0)] = 0u;
-    counters[item_counter(0)] = 0u;
+    counters[rec_counter(0)] = counters[rec_counter(1)] = 0u;
+    counters[item_counter(0)] = counters[item_counter(1)] = 0u;
   }
   if (blockIdx.x * kBlock >= n) return;
   const int ii = i < n ? i : n - 1;
