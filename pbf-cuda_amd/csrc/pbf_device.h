@@ -699,6 +699,25 @@ __device__ __forceinline__ void store_vec(float* __restrict__ a, uint32_t i, flo
   }
 }
 
+// Counts particle of key k into cnt[k] (all lanes of the wavefront call it;
+// valid lanes are a prefix) and returns its arrival number in that cell: one
+// atomic per run of equal keys over consecutive lanes, which get consecutive
+// numbers.
+__device__ __forceinline__ uint32_t count_arrival(uint32_t k, bool valid,
+                                                  uint32_t* __restrict__ cnt) {
+  const int lane = threadIdx.x & 63;
+  const uint32_t prev = __shfl_up(k, 1);
+  const uint64_t vm = __builtin_amdgcn_ballot_w64(valid);
+  const uint64_t hm = __builtin_amdgcn_ballot_w64(valid & ((lane == 0) | (prev != k)));
+  const uint64_t upto = hm & (~0ull >> (63 - lane));
+  const uint64_t later = lane == 63 ? 0ull : (hm >> (lane + 1)) << (lane + 1);
+  const int head = upto ? 63 - __clzll((long long)upto) : lane;
+  const int end = later ? __ffsll((unsigned long long)later) - 1 : __popcll(vm);
+  uint32_t base = 0u;
+  if (valid && lane == head) base = atomicAdd(&cnt[k], (uint32_t)(end - head));
+  return __shfl(base, head) + (uint32_t)(lane - head);
+}
+
 // Particles per cell, counted from the sorted keys (the input of the
 // cell-start scan).  Equal keys are contiguous after the sort, so a run that
 // lies inside one wavefront is that cell's only run and its first lane

@@ -39,9 +39,9 @@ int radix_sort_pairs(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, int
 // the parity-0 counters, each light kernel clears the other parity's).
 void launch_predict_key(int layout, const float* pos, const float* vel, int n, const StepConsts& c,
                         const Scenes& scn, float4* xp, uint32_t* key, uint32_t* val,
-                        uint32_t* counters, hipStream_t st);
+                        uint32_t* counters, uint32_t* cnt, hipStream_t st);
 void launch_key_only(int layout, const float* pos, int n, const StepConsts& c, const Scenes& scn,
-                     float4* xp, uint32_t* key, uint32_t* val, uint32_t* counters,
+                     float4* xp, uint32_t* key, uint32_t* val, uint32_t* counters, uint32_t* cnt,
                      hipStream_t st);
 void launch_fill_u32(uint32_t* a, long long n, uint32_t v, hipStream_t st);
 // Cell-start table from the per-cell counts (which it clears): cs holds
@@ -49,6 +49,26 @@ void launch_fill_u32(uint32_t* a, long long n, uint32_t v, hipStream_t st);
 long long scan_tiles(long long cells);
 void launch_cell_starts(uint32_t* cnt, long long cells, uint32_t* tile_sum, uint32_t* cs,
                         hipStream_t st);
+// Up to how many particles a grid is built by counting (predict / key_only with
+// cnt, then launch_place_ranked) instead of the radix sort (cnt null).  Steps
+// under graph replay, radix -> counted, fresh lattice / dam after 20 frames /
+// after 50: 2K particles 182 / 146 / 147 -> 138 / 106 / 105 us, 128K 477 / 906 /
+// 911 -> 411 / 861 / 875, 512K 886 / 1343 / 1126 -> 825 / 1329 / 1104, 1M 1459 /
+// 2778 / 1860 -> 1387 / 2824 / 1865: there the step's atomics, one per run of
+// equal keys in the previous frame's order, cost what the sort did.  A density
+// error on a finished frame's order has longer runs: 1M 329 / 412 / 262 -> 259 /
+// 396 / 244 (60 frames), 2M 489 / 666 / 523 -> 406 / 636 / 515.
+constexpr int kCountedStepMax = 1 << 19;
+constexpr int kCountedDensityMax = 1 << 21;
+// From the counts cnt and arrival numbers of the predict kernel: the cell-start
+// table cs and the payload in the order of the stable sort; clears cnt.  list:
+// n entries of scratch.  pos null: only xa is moved.  skey, sval (may be null)
+// receive the sorted keys and their input indices.
+void launch_place_ranked(int layout, const uint32_t* key, const uint32_t* arrival, uint2* list,
+                         const float* pos, const float4* xp, const uint32_t* iid, int n,
+                         long long cells, uint32_t* tile_sum, uint32_t* cs, float4* x0s,
+                         float4* xa, uint32_t* iid_s, uint32_t* cnt, uint32_t* skey,
+                         uint32_t* sval, hipStream_t st);
 // The payload gathers after the sort also count the particles per cell from
 // the sorted keys skey into cnt (all zero beforehand), the input of
 // launch_cell_starts.
