@@ -23,8 +23,6 @@
 //  * gather: i sweeps a grid built on the pass's own positions, which holds
 //    every particle within h, and gathers every term that concerns it; no
 //    atomics, every sum in a fixed order.
-#include <utility>
-
 #include "pbf_adjoint.h"
 #include "pbf_pass.h"
 
@@ -560,18 +558,26 @@ __global__ __launch_bounds__(kBlock) void k_bwd_velocity(
   grho[i] = ox.w + ex.w;
 }
 
-// Query cell of position x: written packed (qc, scatter mode) or as the sort
-// key of the pass's grid with its sorted slot (qkey, qval, gather mode).
-__device__ __forceinline__ uint32_t note_query_cell(int i, const float4& x, const StepConsts& c,
+// Query cell of position x: written packed (qc, scatter mode) or as the key of
+// the pass's grid (qkey, gather mode) with, in qval, its sorted slot (the radix
+// sort) or its arrival number in that cell (cnt not null: the counted grid).
+// All lanes of the wavefront call it; invalid ones write nothing.
+__device__ __forceinline__ uint32_t note_query_cell(int i, bool valid, const float4& x,
+                                                    const StepConsts& c,
                                                     uint32_t* __restrict__ qc,
                                                     uint32_t* __restrict__ qkey,
-                                                    uint32_t* __restrict__ qval) {
+                                                    uint32_t* __restrict__ qval,
+                                                    uint32_t* __restrict__ cnt) {
   const Cell q = cell_of(x.x, x.y, x.z, c.g, c.h);
   const uint32_t packed = pack_cell(q);
-  if (qc) qc[i] = packed;
+  if (qc && valid) qc[i] = packed;
   if (qkey) {
-    qkey[i] = cell_id(q, c.g);
-    qval[i] = (uint32_t)i;
+    const uint32_t k = cell_id(q, c.g);
+    const uint32_t v = cnt ? count_arrival(k, valid, cnt) : (uint32_t)i;
+    if (valid) {
+      qkey[i] = k;
+      qval[i] = v;
+    }
   }
   return packed;
 }
@@ -585,22 +591,25 @@ __global__ __launch_bounds__(kBlock) void k_bwd_clamp(
     int n, StepConsts c, const float4* __restrict__ gx, const float4* __restrict__ xl,
     const float4* __restrict__ dp, float4* __restrict__ gxn, float4* __restrict__ A,
     uint32_t* __restrict__ qc, uint32_t* __restrict__ qkey, uint32_t* __restrict__ qval,
-    double* __restrict__ r0, const int* __restrict__ escale) {
+    uint32_t* __restrict__ cnt, double* __restrict__ r0, const int* __restrict__ escale) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (blockIdx.x * kBlock >= n) return;  // whole workgroup past the end
+  const int ii = i < n ? i : n - 1;
+  const float4 x = xl[ii];
+  const uint32_t q = note_query_cell(i, i < n, x, c, qc, qkey, qval, cnt);
   if (i >= n) return;
-  const float4 g = gx[i], x = xl[i], u = dp[i];
+  const float4 g = gx[i], u = dp[i];
   const float gv[3] = {g.x, g.y, g.z}, xv[3] = {x.x, x.y, x.z}, uv[3] = {u.x, u.y, u.z};
   const float lo[3] = {c.g.lox, c.g.loy, c.g.loz}, hi[3] = {c.g.hix, c.g.hiy, c.g.hiz};
   float e[3], a[3];
   double rr = 0.0;
-  for (int q = 0; q < 3; ++q) {
-    const float y = xv[q] + fminf(fmaxf(uv[q], -c.max_dp), c.max_dp);
-    e[q] = (y > lo[q] && y < hi[q]) ? gv[q] : 0.0f;
-    const float db = (uv[q] > -c.max_dp && uv[q] < c.max_dp) ? e[q] : 0.0f;
-    rr += (double)db * (-(double)uv[q] / (double)c.pho0);
-    a[q] = db / c.pho0;
+  for (int d = 0; d < 3; ++d) {
+    const float y = xv[d] + fminf(fmaxf(uv[d], -c.max_dp), c.max_dp);
+    e[d] = (y > lo[d] && y < hi[d]) ? gv[d] : 0.0f;
+    const float db = (uv[d] > -c.max_dp && uv[d] < c.max_dp) ? e[d] : 0.0f;
+    rr += (double)db * (-(double)uv[d] / (double)c.pho0);
+    a[d] = db / c.pho0;
   }
-  const uint32_t q = note_query_cell(i, x, c, qc, qkey, qval);
   gxn[i] = make_float4(e[0], e[1], e[2], 0.0f);
   A[i] = make_float4(a[0], a[1], a[2], __uint_as_float(q));
   r0[i] += escale ? ldexp(rr, *escale) : rr;
@@ -611,10 +620,11 @@ __global__ __launch_bounds__(kBlock) void k_bwd_qcell(int n, StepConsts c,
                                                       const float4* __restrict__ x,
                                                       uint32_t* __restrict__ qc,
                                                       uint32_t* __restrict__ qkey,
-                                                      uint32_t* __restrict__ qval) {
+                                                      uint32_t* __restrict__ qval,
+                                                      uint32_t* __restrict__ cnt) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i >= n) return;
-  note_query_cell(i, x[i], c, qc, qkey, qval);
+  if (blockIdx.x * kBlock >= n) return;
+  note_query_cell(i, i < n, x[i < n ? i : n - 1], c, qc, qkey, qval, cnt);
 }
 
 // Gather mode, once per frame: packed sorted (stale-grid) cell of each
@@ -627,43 +637,69 @@ __global__ __launch_bounds__(kBlock) void k_bwd_sorted_cells(int n, StepConsts c
   pc[i] = pack_cell(cell_of_key(key[i], c.g));
 }
 
-// Gather mode: the inputs of an iteration's delta-p pass in query order
-// (skey: sorted query keys, perm: their sorted slots), with the per-cell
-// counts of the query grid (cnt all zero beforehand).
-__global__ __launch_bounds__(kBlock) void k_bwd_gather_iter(
-    int n, const uint32_t* __restrict__ skey, const uint32_t* __restrict__ perm,
-    const float4* __restrict__ xl, const float4* __restrict__ A, const uint32_t* __restrict__ pc,
-    float4* __restrict__ xq, float4* __restrict__ aq, uint2* __restrict__ cq,
-    uint32_t* __restrict__ cnt) {
-  const int u = blockIdx.x * kBlock + threadIdx.x;
-  if (blockIdx.x * kBlock >= n) return;  // whole workgroup past the end
-  count_sorted(skey, u, n, cnt);
-  if (u >= n) return;
-  const uint32_t s = perm[u] < (uint32_t)n ? perm[u] : 0u;
-  const float4 a = A[s];
-  xq[u] = xl[s];
-  aq[u] = a;
-  cq[u] = make_uint2(pc[s], __float_as_uint(a.w));
+// Gather mode: the query slot and sorted slot of work-item t.  From the radix
+// sort (list null): slot t of the sorted query keys skey, whose sorted slot is
+// perm[t]; counts the particles per cell into cnt (all zero beforehand).  From
+// the counted grid: entry t of list, ranked within its cell; writes perm and
+// clears cnt.  All lanes of the wavefront call it; s is in range for every
+// lane, u only for valid ones.
+struct QuerySlot {
+  uint32_t u, s;
+  bool valid;
+};
+__device__ __forceinline__ QuerySlot query_slot(int n, const uint32_t* __restrict__ skey,
+                                                uint32_t* perm, const uint2* __restrict__ list,
+                                                const uint32_t* __restrict__ cs,
+                                                uint32_t* __restrict__ cnt) {
+  const int t = blockIdx.x * kBlock + threadIdx.x;
+  const bool valid = t < n;
+  if (list) {
+    const uint2 e = list[valid ? t : n - 1];
+    const uint32_t lo = cs[e.y], hi = cs[e.y + 1];
+    const uint32_t u = lo + rank_in_cell(list, lo, hi, e.x, valid);
+    const bool ok = valid && u < (uint32_t)n;  // always, for consistent counts
+    if (ok) {
+      cnt[e.y] = 0u;
+      perm[u] = e.x;
+    }
+    return QuerySlot{u, e.x < (uint32_t)n ? e.x : 0u, ok};
+  }
+  count_sorted(skey, t, n, cnt);
+  const uint32_t s = valid ? perm[t] : 0u;
+  return QuerySlot{(uint32_t)t, s < (uint32_t)n ? s : 0u, valid};
 }
 
-// Gather mode: the inputs of the XSPH pass in query order, with the per-cell
-// counts of the query grid (cnt all zero beforehand).
+// Gather mode: the inputs of an iteration's delta-p pass in query order.
+__global__ __launch_bounds__(kBlock) void k_bwd_gather_iter(
+    int n, const uint32_t* __restrict__ skey, uint32_t* perm, const uint2* __restrict__ list,
+    const uint32_t* __restrict__ cs, const float4* __restrict__ xl, const float4* __restrict__ A,
+    const uint32_t* __restrict__ pc, float4* __restrict__ xq, float4* __restrict__ aq,
+    uint2* __restrict__ cq, uint32_t* __restrict__ cnt) {
+  if (blockIdx.x * kBlock >= n) return;  // whole workgroup past the end
+  const QuerySlot q = query_slot(n, skey, perm, list, cs, cnt);
+  if (!q.valid) return;
+  const float4 a = A[q.s];
+  xq[q.u] = xl[q.s];
+  aq[q.u] = a;
+  cq[q.u] = make_uint2(pc[q.s], __float_as_uint(a.w));
+}
+
+// Gather mode: the inputs of the XSPH pass in query order.
 __global__ __launch_bounds__(kBlock) void k_bwd_gather_xsph(
-    int n, StepConsts c, const uint32_t* __restrict__ skey, const uint32_t* __restrict__ perm,
+    int n, StepConsts c, const uint32_t* __restrict__ skey, uint32_t* perm,
+    const uint2* __restrict__ list, const uint32_t* __restrict__ cs,
     const float4* __restrict__ x, const float4* __restrict__ vr, const float4* __restrict__ gv,
     const uint32_t* __restrict__ pc, float4* __restrict__ xq, float4* __restrict__ vrq,
     float4* __restrict__ gvq, uint2* __restrict__ cq, uint32_t* __restrict__ cnt) {
-  const int u = blockIdx.x * kBlock + threadIdx.x;
   if (blockIdx.x * kBlock >= n) return;  // whole workgroup past the end
-  count_sorted(skey, u, n, cnt);
-  if (u >= n) return;
-  const uint32_t s = perm[u] < (uint32_t)n ? perm[u] : 0u;
-  const float4 p = x[s];
-  const Cell q = cell_of(p.x, p.y, p.z, c.g, c.h);
-  xq[u] = p;
-  vrq[u] = vr[s];
-  gvq[u] = gv[s];
-  cq[u] = make_uint2(pc[s], pack_cell(q));
+  const QuerySlot q = query_slot(n, skey, perm, list, cs, cnt);
+  if (!q.valid) return;
+  const float4 p = x[q.s];
+  const Cell qc = cell_of(p.x, p.y, p.z, c.g, c.h);
+  xq[q.u] = p;
+  vrq[q.u] = vr[q.s];
+  gvq[q.u] = gv[q.s];
+  cq[q.u] = make_uint2(pc[q.s], pack_cell(qc));
 }
 
 // DensityBoundary slope (fluids/Simulator.cu:139-161) at wall distance d.
@@ -852,13 +888,39 @@ void launch_bwd_frame(const BwdFrame& f, int n, const StepConsts& c, hipStream_t
 }
 
 namespace {
-// Gather mode: sorts the sorted slots by the query keys in q.k0 (slots in
-// q.v0) and returns (sorted keys, their sorted slots).
-std::pair<const uint32_t*, const uint32_t*> sort_query(const BwdQuery& q, int n,
-                                                       hipStream_t st) {
+// Gather mode: the query grid of a pass from the keys in q.k0 (with, in q.v0,
+// the sorted slots or the arrival numbers, see note_query_cell), before and
+// after the kernel that gathers the pass's inputs through query_slot.
+struct QueryOrder {
+  const uint32_t* skey = nullptr;
+  uint32_t* perm = nullptr;
+  const uint2* list = nullptr;
+};
+// One frame forward and backward on a stored tape, radix sort -> counted: 32K
+// particles 1101 -> 919 us, 262K 2098 -> 1826, 1M 4971 -> 4662 (fresh lattice) and
+// 7470 -> 7300 (collapsing dam); the 4M sweeping-wall frame 64.0 -> 64.3 ms, its
+// ten grids' atomics costing more than the sort.
+constexpr int kCountedQueryMax = 1 << 20;
+bool counted_query(int n) { return n <= kCountedQueryMax; }
+QueryOrder order_query(const BwdQuery& q, int n, const StepConsts& c, const HeavyLists& hl,
+                       hipStream_t st) {
+  QueryOrder o;
+  if (counted_query(n)) {
+    // the work lists' records are free between neighbour passes
+    uint2* list = reinterpret_cast<uint2*>(hl.recs);
+    launch_count_place(q.k0, q.v0, list, n, c.cells, q.tile_sum, q.cs, q.cnt, st);
+    o.list = list;
+    o.perm = q.v1;
+    return o;
+  }
   const int which =
       radix_sort_pairs(q.k0, q.v0, q.k1, q.v1, n, q.key_bits, q.hist, q.totals, st);
-  return which ? std::make_pair(q.k1, q.v1) : std::make_pair(q.k0, q.v0);
+  o.skey = which ? q.k1 : q.k0;
+  o.perm = which ? q.v1 : q.v0;
+  return o;
+}
+void finish_query(const BwdQuery& q, int n, const StepConsts& c, hipStream_t st) {
+  if (!counted_query(n)) launch_cell_starts(q.cnt, c.cells, q.tile_sum, q.cs, st);
 }
 }  // namespace
 
@@ -866,22 +928,23 @@ void launch_bwd_xsph(const BwdFrame& f, int n, const StepConsts& c, const uint32
                      const HeavyLists& hl, int pass, const Shapes& sh, hipStream_t st) {
   if (f.q) {
     const BwdQuery& q = *f.q;
-    k_bwd_qcell<<<blocks_for(n), kBlock, 0, st>>>(n, c, f.x_final, nullptr, q.k0, q.v0);
-    const auto kv = sort_query(q, n, st);
-    k_bwd_gather_xsph<<<blocks_for(n), kBlock, 0, st>>>(n, c, kv.first, kv.second, f.x_final,
-                                                        f.vr, f.gv_out, q.pc, q.xq, q.vrq,
-                                                        q.gvq, q.cq, q.cnt);
-    launch_cell_starts(q.cnt, c.cells, q.tile_sum, q.cs, st);
+    k_bwd_qcell<<<blocks_for(n), kBlock, 0, st>>>(n, c, f.x_final, nullptr, q.k0, q.v0,
+                                                  counted_query(n) ? q.cnt : nullptr);
+    const QueryOrder o = order_query(q, n, c, hl, st);
+    k_bwd_gather_xsph<<<blocks_for(n), kBlock, 0, st>>>(n, c, o.skey, o.perm, o.list, q.cs,
+                                                        f.x_final, f.vr, f.gv_out, q.pc, q.xq,
+                                                        q.vrq, q.gvq, q.cq, q.cnt);
+    finish_query(q, n, c, st);
     using P = BwdXsphPass<true>;
     launch_pass<P>(P::Args{q.xq, q.vrq, q.gvq, nullptr, f.out_x, f.out_v, nullptr, nullptr,
                            (uint32_t)n, nullptr, q.cq},
                    n, c, Scenes{}, q.cs, hl, pass, sh, st);
-    k_bwd_velocity<true><<<blocks_for(n), kBlock, 0, st>>>(n, c, kv.second, f.gx_out, f.gv_out,
+    k_bwd_velocity<true><<<blocks_for(n), kBlock, 0, st>>>(n, c, o.perm, f.gx_out, f.gv_out,
                                                            f.out_x, f.out_v, nullptr, nullptr,
                                                            f.gx, f.gx0, f.grho_x);
     return;
   }
-  k_bwd_qcell<<<blocks_for(n), kBlock, 0, st>>>(n, c, f.x_final, f.qc, nullptr, nullptr);
+  k_bwd_qcell<<<blocks_for(n), kBlock, 0, st>>>(n, c, f.x_final, f.qc, nullptr, nullptr, nullptr);
   using P = BwdXsphPass<false>;
   launch_pass<P>(P::Args{f.x_final, f.vr, f.gv_out, f.key, f.out_x, f.out_v, f.ex_x, f.ex_v,
                          (uint32_t)n, f.qc, nullptr},
@@ -897,26 +960,27 @@ void launch_bwd_iteration(const BwdFrame& f, const BwdIter& it, int last, int n,
   if (f.q) {
     const BwdQuery& q = *f.q;
     k_bwd_clamp<<<blocks_for(n), kBlock, 0, st>>>(n, c, f.gx, it.xl, it.dp, f.gxn, f.A, nullptr,
-                                                  q.k0, q.v0, f.r0, f.escale);
-    const auto kv = sort_query(q, n, st);
-    k_bwd_gather_iter<<<blocks_for(n), kBlock, 0, st>>>(n, kv.first, kv.second, it.xl, f.A, q.pc,
-                                                        q.xq, q.aq, q.cq, q.cnt);
-    launch_cell_starts(q.cnt, c.cells, q.tile_sum, q.cs, st);
+                                                  q.k0, q.v0, counted_query(n) ? q.cnt : nullptr,
+                                                  f.r0, f.escale);
+    const QueryOrder o = order_query(q, n, c, hl, st);
+    k_bwd_gather_iter<<<blocks_for(n), kBlock, 0, st>>>(n, o.skey, o.perm, o.list, q.cs, it.xl,
+                                                        f.A, q.pc, q.xq, q.aq, q.cq, q.cnt);
+    finish_query(q, n, c, st);
     using PD = BwdDeltaPass<true>;
     launch_pass<PD>(PD::Args{q.xq, q.aq, nullptr, f.out_x, nullptr, (uint32_t)n, q.cq}, n, c,
                     Scenes{}, q.cs, hl, pass, sh, st);
-    k_bwd_lambda_pre<true><<<blocks_for(n), kBlock, 0, st>>>(n, c, last, kv.second, f.out_x,
+    k_bwd_lambda_pre<true><<<blocks_for(n), kBlock, 0, st>>>(n, c, last, o.perm, f.out_x,
                                                              nullptr, it.xl, it.sd, it.rho,
                                                              f.grho_x, f.gxn, q.xr, q.sdb, f.r0,
                                                              f.escale);
     using PL = BwdLambdaPass<true>;
     launch_pass<PL>(PL::Args{q.xr, q.sdb, nullptr, f.gxn, f.gx, nullptr, (uint32_t)n, nullptr,
-                             q.cq, kv.second},
+                             q.cq, o.perm},
                     n, c, Scenes{}, q.cs, hl, pass + 1, sh, st);
     return;
   }
   k_bwd_clamp<<<blocks_for(n), kBlock, 0, st>>>(n, c, f.gx, it.xl, it.dp, f.gxn, f.A, f.qc,
-                                                nullptr, nullptr, f.r0, f.escale);
+                                                nullptr, nullptr, nullptr, f.r0, f.escale);
   using PD = BwdDeltaPass<false>;
   launch_pass<PD>(PD::Args{it.xl, f.A, f.key, f.out_x, f.ex_x, (uint32_t)n, nullptr}, n, c,
                   Scenes{}, cs, hl, pass, sh, st);

@@ -718,6 +718,45 @@ __device__ __forceinline__ uint32_t count_arrival(uint32_t k, bool valid,
   return __shfl(base, head) + (uint32_t)(lane - head);
 }
 
+// Rank of entry i among the cell's entries list[lo, hi).  A cell of up to
+// kRankEntries is read by each of its lanes, eight loads in flight; a larger
+// one (a pile: consecutive slots, so whole wavefronts rank the same cell) by
+// the wavefront together, 64 entries a load, each passed to all lanes.
+constexpr uint32_t kRankEntries = 64;
+__device__ __forceinline__ uint32_t rank_in_cell(const uint2* __restrict__ list, uint32_t lo,
+                                                 uint32_t hi, uint32_t i, bool valid) {
+  const int lane = threadIdx.x & 63;
+  uint32_t rank = 0u;
+  const bool big = valid && hi - lo > kRankEntries;
+  if (valid && !big) {
+    for (uint32_t s = lo; s < hi; s += 8u) {
+      uint32_t e[8];
+#pragma unroll
+      for (int t = 0; t < 8; ++t) e[t] = list[s + t < hi ? s + t : hi - 1u].x;
+#pragma unroll
+      for (int t = 0; t < 8; ++t) rank += ((s + t < hi) & (e[t] < i)) ? 1u : 0u;
+    }
+  }
+  uint64_t todo = __builtin_amdgcn_ballot_w64(big);
+  while (todo) {
+    const int src = __builtin_ctzll(todo);
+    const uint32_t l = (uint32_t)__builtin_amdgcn_readlane((int)lo, src);
+    const uint32_t h = (uint32_t)__builtin_amdgcn_readlane((int)hi, src);
+    const bool mine = big & (lo == l);
+    uint32_t r = 0u;
+    for (uint32_t s = l; s < h; s += 64u) {
+      const uint32_t at = s + (uint32_t)lane;
+      const uint32_t e = at < h ? list[at].x : ~0u;
+#pragma unroll
+      for (int t = 0; t < 64; ++t)
+        r += (uint32_t)__builtin_amdgcn_readlane((int)e, t) < i ? 1u : 0u;
+    }
+    if (mine) rank = r;
+    todo &= ~__builtin_amdgcn_ballot_w64(mine);
+  }
+  return rank;
+}
+
 // Particles per cell, counted from the sorted keys (the input of the
 // cell-start scan).  Equal keys are contiguous after the sort, so a run that
 // lies inside one wavefront is that cell's only run and its first lane

@@ -60,6 +60,12 @@ void launch_cell_starts(uint32_t* cnt, long long cells, uint32_t* tile_sum, uint
 // 396 / 244 (60 frames), 2M 489 / 666 / 523 -> 406 / 636 / 515.
 constexpr int kCountedStepMax = 1 << 19;
 constexpr int kCountedDensityMax = 1 << 21;
+// From the counts cnt and arrival numbers of count_arrival: the cell-start table
+// cs and, listed cell by cell in arrival order, (index, key); the kernel that
+// ranks the list (rank_in_cell) clears cnt.
+void launch_count_place(const uint32_t* key, const uint32_t* arrival, uint2* list, int n,
+                        long long cells, uint32_t* tile_sum, uint32_t* cs, uint32_t* cnt,
+                        hipStream_t st);
 // From the counts cnt and arrival numbers of the predict kernel: the cell-start
 // table cs and the payload in the order of the stable sort; clears cnt.  list:
 // n entries of scratch.  pos null: only xa is moved.  skey, sval (may be null)

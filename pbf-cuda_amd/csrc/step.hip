@@ -695,45 +695,6 @@ __global__ __launch_bounds__(kBlock) void k_place(const uint32_t* __restrict__ k
   if (slot < (uint32_t)n) list[slot] = make_uint2((uint32_t)i, k);  // always, for consistent counts
 }
 
-// Rank of entry i among the cell's entries list[lo, hi).  A cell of up to
-// kRankEntries is read by each of its lanes, eight loads in flight; a larger
-// one (a pile: consecutive slots, so whole wavefronts rank the same cell) by
-// the wavefront together, 64 entries a load, each passed to all lanes.
-constexpr uint32_t kRankEntries = 64;
-__device__ __forceinline__ uint32_t rank_in_cell(const uint2* __restrict__ list, uint32_t lo,
-                                                 uint32_t hi, uint32_t i, bool valid) {
-  const int lane = threadIdx.x & 63;
-  uint32_t rank = 0u;
-  const bool big = valid && hi - lo > kRankEntries;
-  if (valid && !big) {
-    for (uint32_t s = lo; s < hi; s += 8u) {
-      uint32_t e[8];
-#pragma unroll
-      for (int t = 0; t < 8; ++t) e[t] = list[s + t < hi ? s + t : hi - 1u].x;
-#pragma unroll
-      for (int t = 0; t < 8; ++t) rank += ((s + t < hi) & (e[t] < i)) ? 1u : 0u;
-    }
-  }
-  uint64_t todo = __builtin_amdgcn_ballot_w64(big);
-  while (todo) {
-    const int src = __builtin_ctzll(todo);
-    const uint32_t l = (uint32_t)__builtin_amdgcn_readlane((int)lo, src);
-    const uint32_t h = (uint32_t)__builtin_amdgcn_readlane((int)hi, src);
-    const bool mine = big & (lo == l);
-    uint32_t r = 0u;
-    for (uint32_t s = l; s < h; s += 64u) {
-      const uint32_t at = s + (uint32_t)lane;
-      const uint32_t e = at < h ? list[at].x : ~0u;
-#pragma unroll
-      for (int t = 0; t < 64; ++t)
-        r += (uint32_t)__builtin_amdgcn_readlane((int)e, t) < i ? 1u : 0u;
-    }
-    if (mine) rank = r;
-    todo &= ~__builtin_amdgcn_ballot_w64(mine);
-  }
-  return rank;
-}
-
 // L: the caller's layout, or 0 to move xa alone.  Also clears the counts, and
 // on request keeps the sorted keys and the permutation (tapes).
 template <int L>
@@ -911,17 +872,23 @@ void launch_cell_starts(uint32_t* cnt, long long cells, uint32_t* tile_sum, uint
   k_scan_cells<false><<<ntiles, kBlock, 0, st>>>(cnt, cells, tile_sum, cs);
 }
 
-void launch_place_ranked(int layout, const uint32_t* key, const uint32_t* arrival, uint2* list,
-                         const float* pos, const float4* xp, const uint32_t* iid, int n,
-                         long long cells, uint32_t* tile_sum, uint32_t* cs, float4* x0s,
-                         float4* xa, uint32_t* iid_s, uint32_t* cnt, uint32_t* skey,
-                         uint32_t* sval, hipStream_t st) {
+void launch_count_place(const uint32_t* key, const uint32_t* arrival, uint2* list, int n,
+                        long long cells, uint32_t* tile_sum, uint32_t* cs, uint32_t* cnt,
+                        hipStream_t st) {
   const int ntiles = (int)scan_tiles(cells);
   if (ntiles <= kSmallScanTiles)
     k_scan_cells<false, true><<<ntiles, kBlock, 0, st>>>(cnt, cells, nullptr, cs);
   else
     launch_cell_starts(cnt, cells, tile_sum, cs, st);
   k_place<<<blocks_for(n), kBlock, 0, st>>>(key, arrival, n, cs, list);
+}
+
+void launch_place_ranked(int layout, const uint32_t* key, const uint32_t* arrival, uint2* list,
+                         const float* pos, const float4* xp, const uint32_t* iid, int n,
+                         long long cells, uint32_t* tile_sum, uint32_t* cs, float4* x0s,
+                         float4* xa, uint32_t* iid_s, uint32_t* cnt, uint32_t* skey,
+                         uint32_t* sval, hipStream_t st) {
+  launch_count_place(key, arrival, list, n, cells, tile_sum, cs, cnt, st);
   if (!pos)
     k_permute_ranked<0><<<blocks_for(n), kBlock, 0, st>>>(list, cs, nullptr, xp, nullptr, n,
                                                           nullptr, xa, nullptr, cnt, skey, sval);
