@@ -73,15 +73,21 @@ __device__ __forceinline__ int xcd_block_index() {
   return x * per + (x < rem ? x : rem) + (p >> 3);
 }
 
-// The same remap over the first `active` blocks of the grid only (blocks
-// from `active` on get -1).  For a grid-stride kernel whose work fills only a
-// prefix of the grid: remapping over the whole grid would hand that prefix to
-// the first XCDs and leave the others idle.
-__device__ __forceinline__ int xcd_block_index_of(int active) {
-  const int p = (int)blockIdx.x;
-  if (p >= active) return -1;
-  const int per = active >> 3, rem = active & 7, x = p & 7;
-  return x * per + (x < rem ? x : rem) + (p >> 3);
+// Workgroup p of a grid of `grid`, remapped so that each XCD takes runs of kRun
+// consecutive workgroups in turn: neighbours share an L2 as above, and crowded
+// and empty regions fall to all XCDs.  The last, partial round of runs is split
+// evenly (a grid of up to 8 runs: one contiguous range per XCD).
+template <int kRun>
+__device__ __forceinline__ int xcd_runs(int p, int grid) {
+  const int full = grid / (8 * kRun) * (8 * kRun);
+  const int x = p & 7;
+  if (p < full) {
+    const int j = p >> 3;
+    return ((j / kRun) * 8 + x) * kRun + j % kRun;
+  }
+  const int left = grid - full;
+  const int per = left >> 3, rem = left & 7;
+  return full + x * per + (x < rem ? x : rem) + ((p - full) >> 3);
 }
 
 // One axis of the cell coordinate, (int)((p - llim)/h) clamped to
@@ -296,8 +302,7 @@ struct SeqCursor {
   int stride;      // entries apart in LDS
   uint32_t m, b0, c0, n0, b1, n1;
   // With no column after the current one, b1 = n0 makes offsets8 map the
-  // positions past the sequence's end to slots p (< m + 8): in range of a
-  // staged workgroup's padded stage as well as of the particle arrays.
+  // positions past the sequence's end to slots p (< m + 8).
   __device__ __forceinline__ void load_next() {
     if (n0 < m) {
       b1 = e[stride].x;

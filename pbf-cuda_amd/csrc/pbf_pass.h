@@ -14,7 +14,7 @@
 //   finish(a, t, s, c, g) store the result of target t
 // Each neighbour pass is three kernels:
 //   light   one work-item per target over the cell-sorted order; workgroups
-//           remapped so each XCD's L2 serves one contiguous particle range; a
+//           remapped so each XCD's L2 serves runs of neighbouring particles; a
 //           heavy target (pbf_device.h: kLightMax, heavy_level, kLevelShare)
 //           is appended to the heavy list instead;
 //   chunks  one work-item per kChunk-candidate chunk of the heavy targets;
@@ -30,35 +30,24 @@ namespace pbf {
 namespace {
 
 constexpr int kBlock = 256;
+// Workgroups an XCD takes in a row (xcd_runs).  One contiguous range per XCD left
+// the busiest XCD with 1.2 to 1.4 times the mean work (collapsing and spread 1M
+// dam, 4M under the sweeping wall).  Light kernels: runs of 128 workgroups (32K
+// particles, a few x-planes, whose neighbours then share the L2) took the 4M
+// frame from 16.8 to 15.8 ms and the spread 1M step from 1116 to 1080 us, the
+// dense 1M step unchanged; runs of 64 cost that one 1.5%.  Chunk kernels: the
+// list's order already mixes regions and a pile's chunks, all hits, lie
+// together, so short runs: dense 1M step 2575 -> 2413 us with runs of 8 (64:
+// 2424, 1: 2420).
+constexpr int kLightRun = 128;
+constexpr int kChunkRun = 8;
 constexpr int kRankBuckets = 64;  // one wavefront scans them
 // Blocks of 64 candidates whose hits the light kernels evaluate in one loop.
 #ifndef PBF_LIGHT_GROUP
 #define PBF_LIGHT_GROUP 2
 #endif
 constexpr int kLightGroup = PBF_LIGHT_GROUP;
-// A pass policy with kStage = true has its light kernel stage the
-// candidates of each workgroup in LDS (see k_light).  Capacity: kStagePerLane
-// float4 elements per work-item of the workgroup.
-template <class P, class = void>
-struct StageMode {
-  static constexpr bool value = false;
-};
-template <class P>
-struct StageMode<P, std::void_t<decltype(P::kStage)>> {
-  static constexpr bool value = P::kStage;
-};
-// The stage holds x, y and z in three arrays of kStagePerLane * workgroup
-// size + kStagePad floats (a screening batch reads up to 7 elements past the
-// end of a target's last column, masked off).
-#ifndef PBF_STAGE_PER_LANE
-#define PBF_STAGE_PER_LANE 8
-#endif
-constexpr int kStagePerLane = PBF_STAGE_PER_LANE;
-constexpr int kStagePad = 8;
-inline size_t light_lds_bytes(int lb, bool staged) {
-  return (size_t)10 * lb * sizeof(uint2) +
-         (staged ? ((size_t)kStagePerLane * lb + kStagePad) * 12 : 0);
-}
+inline size_t light_lds_bytes(int lb) { return (size_t)kSeqEntries * lb * sizeof(uint2); }
 
 // Minimum wavefronts per SIMD the neighbour kernels are compiled for (caps
 // their registers).
@@ -118,19 +107,13 @@ struct MaskIO {
 template <class P, class S>
 __global__ __launch_bounds__(kBlock, PBF_PASS_WAVES) void k_light(typename P::Args a, int n,
                                                                   StepConsts c, S sc,
-                                                  const uint32_t* __restrict__ cs, HeavyLists hl,
-                                                  int pass, uint32_t fixed_threshold) {
-  constexpr bool kStg = StageMode<P>::value;
+                                                                  const uint32_t* __restrict__ cs,
+                                                                  HeavyLists hl, int pass,
+                                                                  uint32_t fixed_threshold) {
   extern __shared__ uint2 seq_dyn[];
   __shared__ uint32_t key_sh[kBlock];
   __shared__ uint32_t order_sh[kBlock];
   __shared__ uint32_t bucket_sh[kRankBuckets];
-  // staging: per wavefront and column k the smallest first slot and the
-  // largest end slot of its light targets' column k; then per column the
-  // workgroup's range [st_lo, st_lo + size) and its first stage element
-  __shared__ uint32_t wlo_sh[kStg ? kBlock / 64 : 1][9], whi_sh[kStg ? kBlock / 64 : 1][9];
-  __shared__ uint32_t st_lo[9], st_base[10];
-  __shared__ int st_ok;
   uint32_t* rec_cnt = hl.counters + rec_counter(pass & 1);
   uint32_t* item_cnt = hl.counters + item_counter(pass & 1);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -141,25 +124,18 @@ __global__ __launch_bounds__(kBlock, PBF_PASS_WAVES) void k_light(typename P::Ar
   const uint32_t thr = fixed_threshold ? fixed_threshold : (word ? word : kLightMax);
   const int tid = threadIdx.x;
   const int nb = (int)blockDim.x;
-  const int block_base = (P::kXcdRanges ? xcd_block_index() : (int)blockIdx.x) * nb;
+  const int block_base = (P::kXcdRanges ? xcd_runs<kLightRun>((int)blockIdx.x, (int)gridDim.x)
+                                        : (int)blockIdx.x) *
+                         nb;
   const int i = block_base + tid;
   const bool active = i < n;
   const SeqTable st{&seq_dyn[tid], nb};
   typename P::Target t{};
   uint32_t m = 0;
-  Cols cl;
   if (active) {
     t = P::target(a, (uint32_t)i, c);
     const SceneGeo g = sc.at((uint32_t)i, c);
-    const Cell q = cell_of(t.x.x, t.x.y, t.x.z, g, c.h);
-    if constexpr (kStg) {
-      m = load_cols(cl, q, cs, g);
-    } else {
-      m = build_seq(st, q, cs, g);
-    }
-  } else if constexpr (kStg) {
-#pragma unroll
-    for (int k = 0; k < 9; ++k) cl.lo[k] = cl.len[k] = 0u;
+    m = build_seq(st, cell_of(t.x.x, t.x.y, t.x.z, g, c.h), cs, g);
   }
   {
     // this pass's statistics for the next pass's threshold: per level, how
@@ -233,78 +209,11 @@ __global__ __launch_bounds__(kBlock, PBF_PASS_WAVES) void k_light(typename P::Ar
   const uint32_t key = active && (!is_heavy || in_lane) ? m + 1u : 0u;
   key_sh[tid] = key;
   if (tid < kRankBuckets) bucket_sh[tid] = 0u;
-  if constexpr (kStg) {
-    // the workgroup's candidate ranges, column by column, over its light
-    // targets (a heavy target summed in its lane reads global memory)
-    const bool light = active && !is_heavy;
-    const int wave = tid >> 6;
-#pragma unroll
-    for (int k = 0; k < 9; ++k) {
-      const bool has = light && cl.len[k] != 0u;
-      uint32_t lo = has ? cl.lo[k] : 0xFFFFFFFFu;
-      uint32_t hi = has ? cl.lo[k] + cl.len[k] : 0u;
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) {
-        const uint32_t ol = __shfl_xor(lo, off), oh = __shfl_xor(hi, off);
-        lo = ol < lo ? ol : lo;
-        hi = oh > hi ? oh : hi;
-      }
-      if ((tid & 63) == 0) {
-        wlo_sh[wave][k] = lo;
-        whi_sh[wave][k] = hi;
-      }
-    }
-  }
   __syncthreads();
-  if constexpr (kStg) {
-    if (tid == 0) {
-      uint32_t total = 0;
-      for (int k = 0; k < 9; ++k) {
-        uint32_t lo = 0xFFFFFFFFu, hi = 0u;
-        for (int w = 0; w < (nb >> 6); ++w) {
-          lo = wlo_sh[w][k] < lo ? wlo_sh[w][k] : lo;
-          hi = whi_sh[w][k] > hi ? whi_sh[w][k] : hi;
-        }
-        st_lo[k] = lo;
-        st_base[k] = total;
-        total += hi > lo ? hi - lo : 0u;
-      }
-      st_base[9] = total;
-      st_ok = total <= (uint32_t)(kStagePerLane * nb);
-    }
-  }
   const uint32_t bucket =
       key == 0u ? 0u : 1u + min((key - 1u) >> 3, (uint32_t)kRankBuckets - 2u);
   const uint32_t within = atomicAdd(&bucket_sh[bucket], 1u);
   __syncthreads();
-  const uint32_t stage_n = (uint32_t)(kStagePerLane * nb + kStagePad);
-  [[maybe_unused]] float* const stage = reinterpret_cast<float*>(seq_dyn + 10 * nb);
-  if constexpr (kStg) {
-    // column tables: a light target's columns as stage elements when the
-    // workgroup's ranges fit the stage, else (and for a heavy target summed
-    // in its lane) as global slots; then the ranges are copied in,
-    // consecutive work-items taking consecutive elements
-    const bool ok = st_ok != 0;
-    if (active) {
-      const bool staged = ok && !is_heavy;
-      write_seq(st, cl, [&](int k, uint32_t lo) {
-        return staged ? st_base[k] + (lo - st_lo[k]) : lo;
-      });
-    }
-    if (ok) {
-      const uint32_t total = st_base[9];
-      const float4* __restrict__ src_x = P::screen(a);
-      for (uint32_t e = (uint32_t)tid; e < total; e += (uint32_t)nb) {
-        int k = 0;
-#pragma unroll
-        for (int q = 1; q < 9; ++q) k += e >= st_base[q] ? 1 : 0;
-        const float4 v = src_x[st_lo[k] + (e - st_base[k])];
-        stage[e] = v.x;
-        stage[stage_n + e] = v.y;
-        stage[2 * stage_n + e] = v.z;
-      }
-    }
-  }
   if (tid < kRankBuckets) {  // the first wavefront scans the bucket counts
     uint32_t total;
     const uint32_t cnt_b = bucket_sh[tid];
@@ -333,25 +242,6 @@ __global__ __launch_bounds__(kBlock, PBF_PASS_WAVES) void k_light(typename P::Ar
   };
   auto get_mask = [&](uint32_t b, uint64_t& mk) { return mio.get(b, mk); };
   auto put_mask = [&](uint32_t b, uint64_t mk) { mio.put(b, mk); };
-  if constexpr (kStg) {
-    if (st_ok != 0 && ms <= thr) {
-      // the candidates are stage elements (slot = element index); add()
-      // sees the element index as j (pass policies with kStage use j only
-      // for the self test, which their distance test already decides)
-      sweep_seq<P::kHitBatch, kLightGroup>(
-          sts, ms, 0u, ms,
-          [&](uint32_t off) {
-            const uint32_t e = off >> 4;
-            return make_float3(stage[e], stage[stage_n + e], stage[2 * stage_n + e]);
-          },
-          [&](uint32_t j) {
-            return make_float4(stage[j], stage[stage_n + j], stage[2 * stage_n + j], 0.0f);
-          },
-          hit, add, block_end, get_mask, put_mask);
-      P::finish(a, t, s, c, sc.at(ti, c));
-      return;
-    }
-  }
   const Float4Buf sb = float4_buf(P::screen(a), (uint32_t)n);
   // a pass on stored hit masks screens nothing: its hits of up to four
   // blocks run through one loop (kLightMax candidates), which balances the
@@ -375,12 +265,12 @@ __global__ __launch_bounds__(kBlock, PBF_PASS_WAVES) void k_chunks(typename P::A
   const uint32_t items = hl.counters[item_counter(pass & 1)];
   const uint32_t total = items < hl.item_cap ? items : hl.item_cap;
   // only as many workgroups as there are items to go round, spread over all
-  // XCDs, each XCD on one contiguous range of the (chunk-major) item list
+  // XCDs
   const uint32_t need = (total + kBlock - 1) / kBlock;
   const int active = need < gridDim.x ? (int)need : (int)gridDim.x;
-  const int vb = P::kXcdRanges ? xcd_block_index_of(active)
-                               : ((int)blockIdx.x < active ? (int)blockIdx.x : -1);
-  if (vb < 0) return;
+  if ((int)blockIdx.x >= active) return;
+  const int vb =
+      P::kXcdRanges ? xcd_runs<kChunkRun>((int)blockIdx.x, active) : (int)blockIdx.x;
   const uint32_t stride = (uint32_t)active * kBlock;
   const SeqTable st{&seq[0][threadIdx.x], kBlock};
   const Float4Buf sb = float4_buf(P::screen(a), (uint32_t)n);
@@ -500,7 +390,7 @@ void launch_pass_s(const typename P::Args& a, int n, const StepConsts& c, const 
     return;
   }
   const int lb = sh.light_block;
-  k_light<P, S><<<(n + lb - 1) / lb, lb, light_lds_bytes(lb, StageMode<P>::value), st>>>(
+  k_light<P, S><<<(n + lb - 1) / lb, lb, light_lds_bytes(lb), st>>>(
       a, n, c, sc, cs, hl, pass, (uint32_t)sh.heavy);
   k_chunks<P, S><<<grid_for_items(hl.item_cap, sh.chunk_blocks), kBlock, 0, st>>>(a, n, c, sc,
                                                                                     cs, hl, pass);

@@ -35,12 +35,6 @@ namespace {
 struct LambdaPass {
   static constexpr bool kXcdRanges = true;  // one contiguous range per XCD
   static constexpr int kMask = kMaskStore;  // hit masks for the delta-p pass
-  // light workgroups stage their candidates' positions in LDS; add() uses j
-  // only for the self test, which r >= KERNAL_EPS already excludes
-#ifndef PBF_STAGE
-#define PBF_STAGE 0
-#endif
-  static constexpr bool kStage = PBF_STAGE != 0;
   // hits reloaded per round of the sweep
   static constexpr int kHitBatch = 4;
   struct Args {
@@ -83,8 +77,7 @@ struct LambdaPass {
         s.gy = s.gy + ay;
         s.gz = s.gz + az;
         // j != i (Simulator_kernel.cuh:98): i itself has r = 0 < KERNAL_EPS
-        // and never reaches this branch, so no index test is needed (j may
-        // be a stage element index here)
+        // and never reaches this branch, so no index test is needed
         s.gl2 = fmaf(ax, ax, s.gl2);
         s.gl2 = fmaf(ay, ay, s.gl2);
         s.gl2 = fmaf(az, az, s.gl2);
