@@ -99,7 +99,7 @@ struct MaskIO {
 // (64, 128 or 256), the column tables live in dynamic LDS.  A heavy target
 // (more candidates than fixed_threshold, or when that is 0 than the
 // threshold word the previous pass's combine kernel set) gets one chunk item per kChunk candidates and a
-// record, appended with one atomic per wavefront each.  The counters of
+// record, appended with one atomic per workgroup each.  The counters of
 // parity pass & 1 belong to this pass; the kernel clears the other parity's
 // counters for the next pass (their previous users finished earlier on the
 // stream).  If the chunk list is full the lane sums its target itself, still
@@ -114,6 +114,7 @@ __global__ __launch_bounds__(kBlock, PBF_PASS_WAVES) void k_light(typename P::Ar
   __shared__ uint32_t key_sh[kBlock];
   __shared__ uint32_t order_sh[kBlock];
   __shared__ uint32_t bucket_sh[kRankBuckets];
+  __shared__ uint32_t alloc_sh[2][kBlock / 64];
   uint32_t* rec_cnt = hl.counters + rec_counter(pass & 1);
   uint32_t* item_cnt = hl.counters + item_counter(pass & 1);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -157,19 +158,44 @@ __global__ __launch_bounds__(kBlock, PBF_PASS_WAVES) void k_light(typename P::Ar
   }
   const bool is_heavy = active && m > thr;
   const uint32_t nch = is_heavy ? (m + kChunk - 1) / kChunk : 0u;
+  const int wave = tid >> 6;
+  const uint64_t hm = __builtin_amdgcn_ballot_w64(is_heavy);
+  uint32_t item_total = 0u, item_off = 0u;
+  if (hm) item_off = wave_exclusive_sum(nch, &item_total);
+  if ((tid & 63) == 0) {
+    alloc_sh[0][wave] = item_total;
+    alloc_sh[1][wave] = (uint32_t)__popcll(hm);
+  }
+  if (tid < kRankBuckets) bucket_sh[tid] = 0u;
+  __syncthreads();
+  uint32_t heavy = 0u;
+#pragma unroll
+  for (int k = 0; k < kBlock / 64; ++k) heavy += k < (nb >> 6) ? alloc_sh[1][k] : 0u;
   bool in_lane = false;  // chunk list full: this lane sums its chunks itself
-  if (__ballot(is_heavy) != 0ull) {
-    // Wave-aggregated allocation.  Partials are target-major (lane l owns
-    // [first, first + nch)); the work items are chunk-major over the wave
-    // (chunk 0 of every heavy lane, then chunk 1, ...), so the lanes of a
-    // chunk kernel wavefront work on the same chunk of neighbouring targets,
-    // which in a crowded cell share their candidate sequence: the candidate
-    // loads coalesce instead of being gathered lane by lane.
-    uint32_t item_total;
-    const uint32_t item_off = wave_exclusive_sum(nch, &item_total);
-    uint32_t item_base = 0, rec_base = 0;
-    if ((threadIdx.x & 63) == 0) item_base = atomicAdd(item_cnt, item_total);
-    item_base = __shfl(item_base, 0);
+  if (heavy) {
+    // Allocation, one atomic a workgroup and counter: every workgroup's go to
+    // the same two words, where they queue.  (Two a wavefront, one after the
+    // other: 1M dense step 2413 -> 2316 us, 512K dam 1334 -> 1237 us, 64 scenes
+    // 8921 -> 8825 us without them.)  Partials are target-major (lane
+    // l owns [first, first + nch)); the work items are chunk-major over the
+    // wave (chunk 0 of every heavy lane, then chunk 1, ...), so the lanes of
+    // a chunk kernel wavefront work on the same chunk of neighbouring
+    // targets, which in a crowded cell share their candidate sequence: the
+    // candidate loads coalesce instead of being gathered lane by lane.
+    __syncthreads();
+    if (tid < 2) {
+      uint32_t sum = 0u, w[kBlock / 64];
+#pragma unroll
+      for (int k = 0; k < kBlock / 64; ++k) {
+        w[k] = sum;
+        sum += k < (nb >> 6) ? alloc_sh[tid][k] : 0u;
+      }
+      const uint32_t base = atomicAdd(tid ? rec_cnt : item_cnt, sum);
+#pragma unroll
+      for (int k = 0; k < kBlock / 64; ++k) alloc_sh[tid][k] = base + w[k];
+    }
+    __syncthreads();
+    const uint32_t item_base = alloc_sh[0][wave];
     const uint32_t first = item_base + item_off;
     const bool wave_fits = item_base + item_total <= hl.item_cap;
     uint32_t maxnch = nch;
@@ -189,15 +215,10 @@ __global__ __launch_bounds__(kBlock, PBF_PASS_WAVES) void k_light(typename P::Ar
                                 : make_uint4(~0u, 0u, 0u, 0u);
       pos += (uint32_t)__popcll(bm);
     }
-    const uint64_t hm = __ballot(is_heavy);
-    if (wave_fits) {
-      if ((threadIdx.x & 63) == 0) rec_base = atomicAdd(rec_cnt, (uint32_t)__popcll(hm));
-      rec_base = __shfl(rec_base, 0);
-      if (is_heavy)
-        hl.recs[rec_base + (uint32_t)__popcll(hm & lt)] = make_uint4((uint32_t)i, first, nch, 0u);
-    } else {
-      in_lane = is_heavy;
-    }
+    if (is_heavy)  // a record without items is skipped by the combine kernel
+      hl.recs[alloc_sh[1][wave] + (uint32_t)__popcll(hm & lt)] =
+          make_uint4(wave_fits ? (uint32_t)i : ~0u, first, nch, 0u);
+    in_lane = is_heavy && !wave_fits;
   }
   // Lanes take the block's remaining targets in order of candidate count, so
   // each wavefront gets targets of similar cost instead of waiting on its
@@ -208,8 +229,6 @@ __global__ __launch_bounds__(kBlock, PBF_PASS_WAVES) void k_light(typename P::Ar
   // moves, so the order within a bucket (set by LDS atomics) does not matter.
   const uint32_t key = active && (!is_heavy || in_lane) ? m + 1u : 0u;
   key_sh[tid] = key;
-  if (tid < kRankBuckets) bucket_sh[tid] = 0u;
-  __syncthreads();
   const uint32_t bucket =
       key == 0u ? 0u : 1u + min((key - 1u) >> 3, (uint32_t)kRankBuckets - 2u);
   const uint32_t within = atomicAdd(&bucket_sh[bucket], 1u);
@@ -329,6 +348,7 @@ __global__ __launch_bounds__(kBlock) void k_combine(typename P::Args a, int n, S
   const uint32_t stride = gridDim.x * kBlock;
   for (uint32_t r = blockIdx.x * kBlock + threadIdx.x; r < nrec; r += stride) {
     const uint4 rec = hl.recs[r];
+    if (rec.x == ~0u) continue;
     const typename P::Target t = P::target(a, rec.x, c);
     typename P::Acc s;
     using PAcc = typename P::Acc;
