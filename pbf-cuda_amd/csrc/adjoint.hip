@@ -239,6 +239,11 @@ struct BwdXsphPass {
     float dx, dy, dz;
     return dist2(t.x, xj, dx, dy, dz) < c.h2;
   }
+  static constexpr bool kNear = true;
+  static __device__ __forceinline__ float near(const Target& t, const float3& xj,
+                                               const StepConsts& c) {
+    return near2(t.x, xj, c.h2_outer);
+  }
   static __device__ __forceinline__ void add(Acc& s, const Target& t, uint32_t j, const Nb& nb,
                                              const StepConsts& c, const Args& a) {
     float dx, dy, dz;

@@ -148,6 +148,31 @@ constexpr uint32_t kLevelShare = 25;
 constexpr int kLevelBits = 21;
 constexpr int kLevelWords = (kLevels + 2) / 3;
 
+// A pass policy's eight-candidate screening test: the sign bits of near(),
+// negative where the pair may add something, one bit each by a shift of bit
+// pairs, if the policy has it; else its hit().
+template <class P, class T, class = void>
+struct Test8 {
+  static __device__ __forceinline__ uint32_t bits(const T& t, const float3 (&d)[8],
+                                                  const StepConsts& c) {
+    uint32_t b = 0u;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) b |= (P::hit(t, d[k], c) ? 1u : 0u) << k;
+    return b;
+  }
+};
+template <class P, class T>
+struct Test8<P, T, std::void_t<decltype(P::kNear)>> {
+  static __device__ __forceinline__ uint32_t bits(const T& t, const float3 (&d)[8],
+                                                  const StepConsts& c) {
+    uint32_t b = 0u;
+#pragma unroll
+    for (int k = 7; k >= 0; --k)
+      b = __builtin_amdgcn_alignbit(b, __float_as_uint(P::near(t, d[k], c)), 31u);
+    return b;
+  }
+};
+
 // Hit masks shared by the two passes of one solver iteration.  lambda_k and
 // delta-p_k read the same positions x_k and walk the same candidate sequence,
 // and every pair delta-p adds (KERNAL_EPS <= r < h, j != i) passes lambda's
@@ -398,12 +423,13 @@ struct SeqCursor1 {
 };
 
 // The hit mask of the candidates [bb, be) (at most 64, one canonical block)
-// of a target's sequence: eight screening loads in flight at a time, bit
-// u - bb set where hit() holds.  c1 walks forward only.
-template <class LoadS, class Hit>
-__device__ __forceinline__ uint64_t screen_block(SeqCursor& c1, uint32_t bb, uint32_t be,
-                                                 LoadS&& load_s, Hit&& hit) {
-  uint64_t mask = 0;
+// of a target's sequence as two 32-bit words: eight screening loads in flight
+// at a time; test8 turns their eight elements into eight bits.  c1 walks forward only.
+template <class LoadS, class Test8>
+__device__ __forceinline__ void screen_block(SeqCursor& c1, uint32_t bb, uint32_t be,
+                                             LoadS&& load_s, Test8&& test8, uint32_t& lo,
+                                             uint32_t& hi) {
+  lo = hi = 0u;
 #pragma unroll 1
   for (uint32_t u = bb; u < be; u += 8) {
     uint32_t off[8];
@@ -411,90 +437,90 @@ __device__ __forceinline__ uint64_t screen_block(SeqCursor& c1, uint32_t bb, uin
     float3 d[8];
 #pragma unroll
     for (int t = 0; t < 8; ++t) d[t] = load_s(off[t]);
-    uint32_t bits = 0;
-#pragma unroll
-    for (int t = 0; t < 8; ++t) bits |= (hit(d[t]) ? 1u : 0u) << t;
     const uint32_t valid = be - u >= 8u ? 0xFFu : (1u << (be - u)) - 1u;
-    mask |= (uint64_t)(bits & valid) << (u - bb);
+    const uint32_t bits = test8(d) & valid;
+    const uint32_t at = u - bb;  // the same for every lane
+    if (at < 32u)
+      lo |= bits << at;
+    else
+      hi |= bits << (at - 32u);
   }
-  return mask;
 }
 
 // Visits sequence positions [u0, u1) of a candidate sequence of m positions
-// in order,
-// calling add() only for candidates passing the cheap test hit() on their
+// in order, calling add() only for candidates passing the cheap test8 on their
 // x, y, z (load_s(byte offset of the slot's 16-byte element)).  The
-// positions are taken in groups
-// of NB blocks of 64: each block of the group is screened eight loads at a
-// time (across column boundaries, so a sparse neighbourhood costs a few
-// memory round trips, not one or two per column) into a 64-bit hit mask,
-// then the hits of the whole group are reloaded G at a time (a pass
-// policy's kHitBatch) and accumulated in ascending order, with block_end()
-// called once per block, in order, after its last hit.  Running the hits of
-// several blocks through one loop keeps the lanes of a wavefront busy: they
-// wait on the largest hit count of the group instead of that of every
-// block.  Candidates failing hit() contribute exactly nothing in add(), so
-// the sums equal the plain in-order sum.
+// positions are taken in groups of NB blocks of 64: each block of the group
+// is screened eight loads at a time (across column boundaries, so a sparse
+// neighbourhood costs a few memory round trips, not one or two per column)
+// into a hit mask, then the hits of the whole group are reloaded G at a time
+// (a pass policy's kHitBatch) and accumulated in ascending order, with
+// block_end() called after the last hit of each block that has any, in order.
+// Running the hits of several blocks through one loop keeps the lanes of a
+// wavefront busy: they wait on the largest hit count of the group instead of
+// that of every block.  Candidates failing the test contribute exactly
+// nothing in add() (and a block without hits sums to zero), so the sums equal
+// the plain in-order sum.
 // The screening is branch-free after the loads (all eight tests are
 // evaluated and masked), so the compiler keeps the eight loads in flight
 // together instead of sinking some of them into conditional blocks that
-// wait for each load in turn; hit() must be branch-free as well.
-// get_mask(b, mask) may supply block b's hit mask (b = position / 64; u0
-// must be a multiple of 64) instead of screening it; put_mask(b, mask)
+// wait for each load in turn; the tests must be branch-free as well.
+// The masks are walked as 32-bit words, the first of which holds the next hit:
+// a hit costs one find-first, one clear and one select per word, where 64-bit
+// masks took twice the instructions (a lane whose next word is empty sits one
+// hit out).
+// get_mask(b, lo, hi) may supply block b's hit mask (b = position / 64; u0
+// must be a multiple of 64) instead of screening it; put_mask(b, lo, hi)
 // receives each mask the sweep screened.
-template <int G, int NB, class LoadS, class LoadF, class Hit, class Add, class BlockEnd,
+template <int G, int NB, class LoadS, class LoadF, class Test8, class Add, class BlockEnd,
           class GetMask, class PutMask>
 __device__ __forceinline__ void sweep_seq(const SeqTable& st, uint32_t m, uint32_t u0,
                                           uint32_t u1, LoadS&& load_s, LoadF&& load_f,
-                                          Hit&& hit, Add&& add, BlockEnd&& block_end,
+                                          Test8&& test8, Add&& add, BlockEnd&& block_end,
                                           GetMask&& get_mask, PutMask&& put_mask) {
   if (u0 >= u1) return;
+  constexpr int NW = 2 * NB;
   SeqCursor c1;
   c1.init(st, u0, m);
   SeqCursor1 c2;
   c2.from(c1);
 #pragma unroll 1
   for (uint32_t gb = u0; gb < u1; gb += 64u * NB) {
-    uint64_t w[NB];
+    uint32_t w[NW];
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
       const uint32_t bb = gb + 64u * (uint32_t)q;
-      uint64_t mask = 0;
-      if (bb < u1 && !get_mask(bb >> 6, mask)) {
+      w[2 * q] = w[2 * q + 1] = 0u;
+      if (bb < u1 && !get_mask(bb >> 6, w[2 * q], w[2 * q + 1])) {
         const uint32_t be = u1 - bb < 64u ? u1 : bb + 64u;
-        mask = screen_block(c1, bb, be, load_s, hit);
-        put_mask(bb >> 6, mask);
+        screen_block(c1, bb, be, load_s, test8, w[2 * q], w[2 * q + 1]);
+        put_mask(bb >> 6, w[2 * q], w[2 * q + 1]);
       }
-      w[q] = mask;
     }
-    const uint32_t left = (u1 - gb + 63u) >> 6;
-    const uint32_t nblk = left < (uint32_t)NB ? left : (uint32_t)NB;
-    // the hits of the group: w[0] holds block q's remaining hits (the words
-    // move down as blocks run out)
-    uint32_t q = 0, done = 0, last = gb;
+    // w[0] holds the remaining hits of positions [base, base + 32); block: the
+    // one being summed
+    uint32_t base = gb, last = gb, block = gb >> 6;
 #pragma unroll 1
     while (true) {
-      uint64_t any = w[0];
+      uint32_t any = w[0];
 #pragma unroll
-      for (int k = 1; k < NB; ++k) any |= w[k];
+      for (int k = 1; k < NW; ++k) any |= w[k];
       if (!any) break;
-      uint32_t j[G], qt[G];
+      uint32_t j[G], blk[G];
       bool h[G];
 #pragma unroll
       for (int t = 0; t < G; ++t) {
-        while (w[0] == 0u && q + 1u < nblk) {
+        const bool used = w[0] == 0u;
 #pragma unroll
-          for (int k = 0; k + 1 < NB; ++k) w[k] = w[k + 1];
-          w[NB - 1] = 0u;
-          ++q;
-        }
+        for (int k = 0; k < NW; ++k) w[k] = used ? (k + 1 < NW ? w[k + 1] : 0u) : w[k];
+        base += used ? 32u : 0u;
         h[t] = w[0] != 0u;
-        // past the last hit, repeat it (the cursor only moves forward)
-        const uint32_t pos = h[t] ? gb + 64u * q + (uint32_t)__builtin_ctzll(w[0]) : last;
+        // no hit: repeat the last (the cursor only moves forward)
+        const uint32_t pos = h[t] ? base + (uint32_t)__builtin_ctz(w[0]) : last;
         last = pos;
         w[0] &= w[0] - 1u;
         j[t] = c2.slot(pos);
-        qt[t] = q;
+        blk[t] = base >> 6;
       }
       decltype(load_f(0u)) d[G];
 #pragma unroll
@@ -502,17 +528,14 @@ __device__ __forceinline__ void sweep_seq(const SeqTable& st, uint32_t m, uint32
 #pragma unroll
       for (int t = 0; t < G; ++t)
         if (h[t]) {
-          while (done < qt[t]) {
+          if (NB > 1 && blk[t] != block) {
             block_end();
-            ++done;
+            block = blk[t];
           }
           add(j[t], d[t]);
         }
     }
-    while (done < nblk) {
-      block_end();
-      ++done;
-    }
+    block_end();
   }
 }
 
@@ -615,6 +638,13 @@ __device__ __forceinline__ float dist2(const float4& a, const float3& b, float& 
   r2 = fmaf(dy, dy, r2);
   r2 = fmaf(dz, dz, r2);
   return r2;
+}
+
+// |a - b|^2 - bound with the bound as the first addend: negative below it, up to
+// rounding (~1e-7 of the bound).
+__device__ __forceinline__ float near2(const float4& a, const float3& b, float bound) {
+  const float dx = a.x - b.x, dy = a.y - b.y, dz = a.z - b.z;
+  return fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, -bound)));
 }
 
 // x, y, z of element j of a float4 array (a 12-byte load).

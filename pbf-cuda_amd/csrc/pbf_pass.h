@@ -9,6 +9,8 @@
 //   load_f(a, j)         candidate data for the pair term
 //   hit(t, d, c)         cheap test on the candidate's x, y, z d: false only
 //                        if the pair adds exactly 0 (i itself has d == t.x)
+//   near(t, d, c)        (with kNear) the same as the sign of a number: it may
+//                        be positive or zero only if the pair adds exactly 0
 //   add(acc, t, j, d, c, a) the pair term (the body of the reference's loop)
 //   accumulate(tot, p)   tot += a chunk's partial sum
 //   finish(a, t, s, c, g) store the result of target t
@@ -76,18 +78,20 @@ struct MaskIO {
   __device__ __forceinline__ bool kept() const {
     return hl.masks != nullptr && m <= kMaskBlocks * kChunk;
   }
-  __device__ __forceinline__ bool get(uint32_t b, uint64_t& mask) const {
+  __device__ __forceinline__ bool get(uint32_t b, uint32_t& lo, uint32_t& hi) const {
     if constexpr (MaskMode<P>::value == kMaskLoad) {
       if (kept()) {
-        mask = hl.masks[(size_t)b * hl.mask_stride + ti];
+        const uint64_t mask = hl.masks[(size_t)b * hl.mask_stride + ti];
+        lo = (uint32_t)mask;
+        hi = (uint32_t)(mask >> 32);
         return true;
       }
     }
     return false;
   }
-  __device__ __forceinline__ void put(uint32_t b, uint64_t mask) const {
+  __device__ __forceinline__ void put(uint32_t b, uint32_t lo, uint32_t hi) const {
     if constexpr (MaskMode<P>::value == kMaskStore) {
-      if (kept()) hl.masks[(size_t)b * hl.mask_stride + ti] = mask;
+      if (kept()) hl.masks[(size_t)b * hl.mask_stride + ti] = ((uint64_t)hi << 32) | lo;
     }
   }
 };
@@ -248,7 +252,7 @@ __global__ __launch_bounds__(kBlock, PBF_PASS_WAVES) void k_light(typename P::Ar
   const uint32_t ti = (uint32_t)(block_base + src);
   const SeqTable sts{&seq_dyn[src], nb};
   t = P::target(a, ti, c);
-  auto hit = [&](const float3& d) { return P::hit(t, d, c); };
+  auto test8 = [&](const float3 (&d)[8]) { return Test8<P, typename P::Target>::bits(t, d, c); };
   // the sweep's blocks are the canonical chunks: each is summed from zero
   // and added to the total in order (also for a heavy target whose chunk
   // list was full)
@@ -259,8 +263,8 @@ __global__ __launch_bounds__(kBlock, PBF_PASS_WAVES) void k_light(typename P::Ar
     P::accumulate(s, part);
     part = typename P::Acc{};
   };
-  auto get_mask = [&](uint32_t b, uint64_t& mk) { return mio.get(b, mk); };
-  auto put_mask = [&](uint32_t b, uint64_t mk) { mio.put(b, mk); };
+  auto get_mask = [&](uint32_t b, uint32_t& lo, uint32_t& hi) { return mio.get(b, lo, hi); };
+  auto put_mask = [&](uint32_t b, uint32_t lo, uint32_t hi) { mio.put(b, lo, hi); };
   const Float4Buf sb = float4_buf(P::screen(a), (uint32_t)n);
   // a pass on stored hit masks screens nothing: its hits of up to four
   // blocks run through one loop (kLightMax candidates), which balances the
@@ -268,7 +272,7 @@ __global__ __launch_bounds__(kBlock, PBF_PASS_WAVES) void k_light(typename P::Ar
   constexpr int kGroup = MaskMode<P>::value == kMaskLoad ? (int)(kLightMax / kChunk) : kLightGroup;
   sweep_seq<P::kHitBatch, kGroup>(
       sts, ms, 0u, ms, [&](uint32_t off) { return load_xyz_at(sb, off); },
-      [&](uint32_t j) { return P::load_f(a, j); }, hit, add, block_end, get_mask, put_mask);
+      [&](uint32_t j) { return P::load_f(a, j); }, test8, add, block_end, get_mask, put_mask);
   P::finish(a, t, s, c, sc.at(ti, c));
 }
 
@@ -306,10 +310,10 @@ __global__ __launch_bounds__(kBlock, PBF_PASS_WAVES) void k_chunks(typename P::A
     sweep_seq<P::kHitBatch, 1>(
         st, m, s0, s1, [&](uint32_t off) { return load_xyz_at(sb, off); },
         [&](uint32_t j) { return P::load_f(a, j); },
-        [&](const float3& d) { return P::hit(t, d, c); },
+        [&](const float3 (&d)[8]) { return Test8<P, typename P::Target>::bits(t, d, c); },
         [&](uint32_t j, const auto& d) { P::add(part, t, j, d, c, a); }, [] {},
-        [&](uint32_t b, uint64_t& mk) { return mio.get(b, mk); },
-        [&](uint32_t b, uint64_t mk) { mio.put(b, mk); });
+        [&](uint32_t b, uint32_t& lo, uint32_t& hi) { return mio.get(b, lo, hi); },
+        [&](uint32_t b, uint32_t lo, uint32_t hi) { mio.put(b, lo, hi); });
     *reinterpret_cast<typename P::Acc*>(hl.partials + (size_t)it.z * partial_words<P>()) = part;
   }
 }

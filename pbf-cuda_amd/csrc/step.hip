@@ -60,6 +60,11 @@ struct LambdaPass {
     float dx, dy, dz;
     return dist2(t.x, xj, dx, dy, dz) < c.h2_outer;
   }
+  static constexpr bool kNear = true;
+  static __device__ __forceinline__ float near(const Target& t, const float3& xj,
+                                               const StepConsts& c) {
+    return near2(t.x, xj, c.h2_outer);
+  }
   static __device__ __forceinline__ void add(Acc& s, const Target& t, uint32_t j, const float4& xj,
                                              const StepConsts& c, const Args&) {
     float dx, dy, dz;
@@ -306,6 +311,11 @@ struct XsphPass {
     float dx, dy, dz;
     return dist2(t.x, xj, dx, dy, dz) < c.h2;
   }
+  static constexpr bool kNear = true;
+  static __device__ __forceinline__ float near(const Target& t, const float3& xj,
+                                               const StepConsts& c) {
+    return near2(t.x, xj, c.h2_outer);
+  }
   static __device__ __forceinline__ void add(Acc& s, const Target& t, uint32_t, const Nb& nb,
                                              const StepConsts& c, const Args&) {
     float dx, dy, dz;
@@ -378,6 +388,11 @@ struct DensityPass {
                                              const StepConsts& c) {
     float dx, dy, dz;
     return dist2(t.x, xj, dx, dy, dz) < c.h2;
+  }
+  static constexpr bool kNear = true;
+  static __device__ __forceinline__ float near(const Target& t, const float3& xj,
+                                               const StepConsts& c) {
+    return near2(t.x, xj, c.h2_outer);
   }
   static __device__ __forceinline__ void add(Acc& s, const Target& t, uint32_t, const float4& xj,
                                              const StepConsts& c, const Args&) {
