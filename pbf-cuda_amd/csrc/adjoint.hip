@@ -193,6 +193,7 @@ struct BwdXsphPass {
   // crowded cell's targets scatter from all eight XCDs, each into its own
   // copy; gather mode: one contiguous range per XCD
   static constexpr bool kXcdRanges = kGather;
+  static constexpr bool kCoarse = kGather;
   // hits reloaded per round of the sweep
   static constexpr int kHitBatch = 4;
   struct Args {
@@ -695,13 +696,15 @@ __global__ __launch_bounds__(kBlock) void k_bwd_gather_xsph(
     const uint2* __restrict__ list, const uint32_t* __restrict__ cs,
     const float4* __restrict__ x, const float4* __restrict__ vr, const float4* __restrict__ gv,
     const uint32_t* __restrict__ pc, float4* __restrict__ xq, float4* __restrict__ vrq,
-    float4* __restrict__ gvq, uint2* __restrict__ cq, uint32_t* __restrict__ cnt) {
+    float4* __restrict__ gvq, uint2* __restrict__ cq, uint2* __restrict__ coarse,
+    uint32_t* __restrict__ cnt) {
   if (blockIdx.x * kBlock >= n) return;  // whole workgroup past the end
   const QuerySlot q = query_slot(n, skey, perm, list, cs, cnt);
   if (!q.valid) return;
   const float4 p = x[q.s];
   const Cell qc = cell_of(p.x, p.y, p.z, c.g, c.h);
   xq[q.u] = p;
+  if (coarse) coarse[q.u] = screen_coords(p.x, p.y, p.z, c);
   vrq[q.u] = vr[q.s];
   gvq[q.u] = gv[q.s];
   cq[q.u] = make_uint2(pc[q.s], pack_cell(qc));
@@ -938,7 +941,8 @@ void launch_bwd_xsph(const BwdFrame& f, int n, const StepConsts& c, const uint32
     const QueryOrder o = order_query(q, n, c, hl, st);
     k_bwd_gather_xsph<<<blocks_for(n), kBlock, 0, st>>>(n, c, o.skey, o.perm, o.list, q.cs,
                                                         f.x_final, f.vr, f.gv_out, q.pc, q.xq,
-                                                        q.vrq, q.gvq, q.cq, q.cnt);
+                                                        q.vrq, q.gvq, q.cq,
+                                                        coarse_of(hl, n, sh), q.cnt);
     finish_query(q, n, c, st);
     using P = BwdXsphPass<true>;
     launch_pass<P>(P::Args{q.xq, q.vrq, q.gvq, nullptr, f.out_x, f.out_v, nullptr, nullptr,

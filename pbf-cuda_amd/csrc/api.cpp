@@ -339,6 +339,7 @@ int make_consts(pbf_solver* s, const pbf_params& p, pbf_vec3 ul, pbf_vec3 ll,
   c.inv_dt = 1.0f / p.dt;  // h_updateVelocity, fluids/Simulator.cu:129
   c.gz = -p.g;
   c.c_xsph = p.c_XSPH;
+  c.inv_screen = 1.0 / (16.0 * (double)p.h);
   return PBF_OK;
 }
 
@@ -477,6 +478,7 @@ void enqueue_step(pbf_solver* s, const StepArrays& a, const pbf::StepConsts& c, 
   tb(PBF_PHASE_STEP);
   // advect() + getGridId (Simulator.cpp:50, Simulator.cu:165-193)
   const bool counted = n <= pbf::kCountedStepMax;
+  uint2* const coarse = pbf::coarse_of(s->hl, n, sh);
   tb(PBF_PHASE_PREDICT);
   pbf::launch_predict_key(L, a.pos, a.vel, n, c, scn, s->xp, s->key0, s->val0, s->counters,
                           counted ? s->cnt : nullptr, st);
@@ -486,8 +488,8 @@ void enqueue_step(pbf_solver* s, const StepArrays& a, const pbf::StepConsts& c, 
   if (counted) {
     // the work lists' records are free until the first neighbour pass
     tb(PBF_PHASE_GRID);
-    pbf::launch_place_ranked(L, s->key0, s->val0, (uint2*)s->hl.recs, a.pos, s->xp, a.iid, n,
-                             c.cells, s->tile_sum, s->cs, s->x0s, s->xa, s->iid_s, s->cnt,
+    pbf::launch_place_ranked(L, s->key0, s->val0, (uint2*)s->hl.recs, a.pos, s->xp, a.iid, n, c,
+                             s->tile_sum, s->cs, s->x0s, s->xa, coarse, s->iid_s, s->cnt,
                              rec ? s->key1 : nullptr, rec ? s->val1 : nullptr, st);
     te(PBF_PHASE_GRID);
     if (rec) {
@@ -508,8 +510,8 @@ void enqueue_step(pbf_solver* s, const StepArrays& a, const pbf::StepConsts& c, 
     // the payload gather counts the particles per cell, the scan turns the
     // counts into cell starts
     tb(PBF_PHASE_GRID);
-    pbf::launch_permute(L, skey, sval, a.pos, s->xp, a.iid, n, s->x0s, s->xa, s->iid_s, s->cnt,
-                        st);
+    pbf::launch_permute(L, skey, sval, a.pos, s->xp, a.iid, n, c, s->x0s, s->xa, coarse,
+                        s->iid_s, s->cnt, st);
     pbf::launch_cell_starts(s->cnt, c.cells, s->tile_sum, s->cs, st);
     te(PBF_PHASE_GRID);
   }
@@ -647,7 +649,7 @@ int find_or_record(pbf_solver* s, const StepArrays& a, const pbf::StepConsts& c,
 // particles, `max_cells` cells and `nscenes` scenes (0: a single scene).
 struct ArenaLayout {
   size_t key0, val0, key1, val1, iid, hist, tot, xp, x0s, xa, vr, rho, recs, items, part, cnt,
-      de, dp, dout, cnt2, cs, ts, geo, sid, mask;
+      de, dp, dout, cnt2, cs, ts, geo, sid, mask, coarse;
   size_t icap, total;
 };
 
@@ -693,6 +695,7 @@ ArenaLayout arena_layout(int capacity, long long max_cells, int nscenes) {
   L.geo = carve(sizeof(pbf::SceneGeo) * (size_t)(nscenes > 0 ? nscenes : 1));
   L.sid = carve(nscenes > 0 ? 2 * N : 2);
   L.mask = carve(8 * pbf::kMaskBlocks * N);
+  L.coarse = carve(8 * N);
   L.total = off;
   return L;
 }
@@ -720,6 +723,7 @@ void bind_arena(pbf_solver* s, char* b, const ArenaLayout& L, int capacity) {
   s->hl.item_cap = (uint32_t)L.icap;
   s->hl.masks = (uint64_t*)(b + L.mask);
   s->hl.mask_stride = (uint32_t)capacity;
+  s->hl.coarse = (uint2*)(b + L.coarse);
   s->dens_err = (double*)(b + L.de);
   s->dens_partial = (double*)(b + L.dp);
   s->dens_out = (double*)(b + L.dout);
@@ -1294,17 +1298,18 @@ int pbf_density_error(pbf_solver* s, const float* pos, int n, void* stream, doub
   if (s->cnt_dirty) pbf::launch_fill_u32(s->cnt, s->max_cells, 0u, st);
   s->cnt_dirty = true;
   const bool counted = n <= pbf::kCountedDensityMax;
+  uint2* const coarse = pbf::coarse_of(s->hl, n, s->shapes);
   pbf::launch_key_only(s->layout, pos, n, c, scn, s->xp, s->key0, s->val0, s->counters,
                        counted ? s->cnt : nullptr, st);
   if (counted) {
     pbf::launch_place_ranked(s->layout, s->key0, s->val0, (uint2*)s->hl.recs, nullptr, s->xp,
-                             nullptr, n, c.cells, s->tile_sum, s->cs, nullptr, s->xa, nullptr,
+                             nullptr, n, c, s->tile_sum, s->cs, nullptr, s->xa, coarse, nullptr,
                              s->cnt, nullptr, nullptr, st);
   } else {
     const int which = pbf::radix_sort_pairs(s->key0, s->val0, s->key1, s->val1, n,
                                             key_bits_for(c.cells), s->hist, s->totals, st);
-    pbf::launch_permute_pos(which ? s->key1 : s->key0, which ? s->val1 : s->val0, s->xp, n, s->xa,
-                            s->cnt, st);
+    pbf::launch_permute_pos(which ? s->key1 : s->key0, which ? s->val1 : s->val0, s->xp, n, c,
+                            s->xa, coarse, s->cnt, st);
     pbf::launch_cell_starts(s->cnt, c.cells, s->tile_sum, s->cs, st);
   }
   pbf::launch_density_error(s->xa, s->cs, n, c, scn, s->dens_err, s->dens_partial, s->dens_out,

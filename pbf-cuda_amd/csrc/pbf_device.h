@@ -45,6 +45,7 @@ struct StepConsts {
   float dt, inv_dt;        // dt, 1/dt (FP32, as h_updateVelocity)
   float gz;                // -g
   float c_xsph;
+  double inv_screen;       // 1 / (16 h): periods of the screening coordinates per unit
 };
 
 // Scene sources: where a kernel finds the geometry of particle i's scene.
@@ -148,31 +149,6 @@ constexpr uint32_t kLevelShare = 25;
 constexpr int kLevelBits = 21;
 constexpr int kLevelWords = (kLevels + 2) / 3;
 
-// A pass policy's eight-candidate screening test: the sign bits of near(),
-// negative where the pair may add something, one bit each by a shift of bit
-// pairs, if the policy has it; else its hit().
-template <class P, class T, class = void>
-struct Test8 {
-  static __device__ __forceinline__ uint32_t bits(const T& t, const float3 (&d)[8],
-                                                  const StepConsts& c) {
-    uint32_t b = 0u;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) b |= (P::hit(t, d[k], c) ? 1u : 0u) << k;
-    return b;
-  }
-};
-template <class P, class T>
-struct Test8<P, T, std::void_t<decltype(P::kNear)>> {
-  static __device__ __forceinline__ uint32_t bits(const T& t, const float3 (&d)[8],
-                                                  const StepConsts& c) {
-    uint32_t b = 0u;
-#pragma unroll
-    for (int k = 7; k >= 0; --k)
-      b = __builtin_amdgcn_alignbit(b, __float_as_uint(P::near(t, d[k], c)), 31u);
-    return b;
-  }
-};
-
 // Hit masks shared by the two passes of one solver iteration.  lambda_k and
 // delta-p_k read the same positions x_k and walk the same candidate sequence,
 // and every pair delta-p adds (KERNAL_EPS <= r < h, j != i) passes lambda's
@@ -209,8 +185,7 @@ __device__ pbf_f32x4 pbf_raw_buffer_load_f32x4(pbf_i32x4 rsrc, int voffset, int 
 struct Float4Buf {
   pbf_i32x4 r;
 };
-__device__ __forceinline__ Float4Buf float4_buf(const float4* p, uint32_t n) {
-  const uint64_t bytes = (uint64_t)n * 16u;
+__device__ __forceinline__ Float4Buf raw_buf(const void* p, uint64_t bytes) {
   const uint64_t a = (uint64_t)p;
   Float4Buf b;
   b.r.x = (int)(uint32_t)(a & 0xFFFFFFFFull);
@@ -218,6 +193,9 @@ __device__ __forceinline__ Float4Buf float4_buf(const float4* p, uint32_t n) {
   b.r.z = (int)(bytes > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)bytes);
   b.r.w = 0x00020000;  // the raw (untyped) buffer format of gfx9
   return b;
+}
+__device__ __forceinline__ Float4Buf float4_buf(const float4* p, uint32_t n) {
+  return raw_buf(p, (uint64_t)n * 16u);
 }
 // x, y, z of the element at byte offset `off` (a 12-byte load).
 __device__ __forceinline__ float3 load_xyz_at(const Float4Buf& b, uint32_t off) {
@@ -229,6 +207,40 @@ __device__ __forceinline__ float3 load_xyz_at(const Float4Buf& b, uint32_t off) 
 __device__ __forceinline__ float4 load_f4_at(const Float4Buf& b, uint32_t off) {
   const pbf_f32x4 v = pbf_raw_buffer_load_f32x4(b.r, (int)off, 0, 0);
   return make_float4(v.x, v.y, v.z, v.w);
+}
+
+typedef int pbf_i32x2 __attribute__((ext_vector_type(2)));
+__device__ pbf_i32x2 pbf_raw_buffer_load_i32x2(pbf_i32x4 rsrc, int voffset, int soffset,
+                                               int aux) __asm("llvm.amdgcn.raw.buffer.load.v2i32");
+__device__ pbf_i32x4 pbf_raw_buffer_load_i32x4(pbf_i32x4 rsrc, int voffset, int soffset,
+                                               int aux) __asm("llvm.amdgcn.raw.buffer.load.v4i32");
+
+// Screening coordinates of a position: x | y << 16 and z, each in units of
+// h / 4096 modulo 2^16 (a period of 16 h), formed in FP64 and rounded down.  A
+// candidate then takes 8 bytes and four integer instructions to screen
+// instead of 12 bytes (in a 16-byte element) and six: the differences wrap
+// into [-8 h, 8 h), and a pair closer than h differs by less than 4096 + 1 units
+// per axis from its true difference, so its squared length stays below
+// kScreenNear.  Pairs that alias modulo 16 h or lie just beyond h pass the test
+// too; add() decides those exactly.
+__device__ __forceinline__ uint32_t screen_coord(float x, double inv) {
+  const double t = (double)x * inv;
+  return (uint32_t)((t - floor(t)) * 65536.0) & 0xFFFFu;
+}
+__device__ __forceinline__ uint2 screen_coords(float x, float y, float z, const StepConsts& c) {
+  return make_uint2(screen_coord(x, c.inv_screen) | screen_coord(y, c.inv_screen) << 16,
+                    screen_coord(z, c.inv_screen));
+}
+// (h (1 + 1e-4) in units + sqrt(3) for the rounding of both ends)^2, rounded up
+constexpr int kScreenNear = 4099 * 4099;
+// Squared screening distance minus kScreenNear: negative for every pair within
+// h (whose squares do not overflow).
+__device__ __forceinline__ int screen_near(const uint2& a, const uint2& b) {
+  typedef short s16x2 __attribute__((ext_vector_type(2)));
+  const s16x2 dxy = __builtin_bit_cast(s16x2, a.x) - __builtin_bit_cast(s16x2, b.x);
+  const s16x2 dz = __builtin_bit_cast(s16x2, a.y) - __builtin_bit_cast(s16x2, b.y);
+  return __builtin_amdgcn_sdot2(dz, dz, __builtin_amdgcn_sdot2(dxy, dxy, -kScreenNear, false),
+                                false);
 }
 
 // Entries of a column table: nine columns and the closing entry.
@@ -245,6 +257,22 @@ struct SeqTable {
   __device__ __forceinline__ uint2 at(int k) const { return tab[k * stride]; }
 };
 
+// The cell-start table of a grid as the neighbour passes read it: a column's
+// entries by one 16-byte load, or (apart) its two ends by a load each.  One load
+// is half the cache accesses (1M dense step 2197 -> 2155 us, spread 1075 -> 1056
+// us), but where a pass waits on latency it is the slower one (130,000
+// particles 597 -> 609 us), and it cannot reach 2^30 cells.
+constexpr int kJoinedStartsMin = (1 << 19) + 1;  // particles
+struct CellStarts {
+  const uint32_t* __restrict__ cs;
+  Float4Buf buf;
+  bool apart;
+};
+__device__ __forceinline__ CellStarts cell_starts(const uint32_t* cs, int cells, int n) {
+  return CellStarts{cs, raw_buf(cs, ((uint64_t)(uint32_t)cells + 1u) * 4u),
+                    n < kJoinedStartsMin || (uint32_t)cells >= 1u << 30};
+}
+
 // Candidate neighbours of a particle whose query cell is q, in the
 // reference's order (fluids/Simulator_kernel.cuh:78-88): dx, then dy, then
 // dz, j ascending.  The three cells (x,y,z-1..z+1) of one column are
@@ -252,33 +280,42 @@ struct SeqTable {
 // read from the cell-start table cs (cells + 1 entries; cs[c] = first sorted
 // slot whose cell id is >= c): [cs[first cell], cs[last cell + 1]).  Walking
 // that range is the same j sequence as walking the three cells in turn.
-// build_seq builds the table from the nine column ranges around query cell q
-// (column k = 3*(dx+1) + (dy+1); outside the grid: empty) and returns the
-// candidate count m.  The 18 cell-start loads are issued
-// together (a column outside the grid reads a valid dummy address and is
-// then treated as empty), so building the table costs one memory round trip,
-// not one per column.
-// The nine candidate columns of query cell q as (first slot, length), length
-// 0 for a column outside the grid or empty; the 18 cell-start loads are
-// issued together.
+// The nine candidate columns of query cell q (column k = 3*(dx+1) + (dy+1))
+// as (first slot, length), length 0 for a column outside the grid or empty
+// (outside: a valid dummy address is read); returns the candidate count m.
+// The loads of all columns are issued together: one memory round trip.
 struct Cols {
   uint32_t lo[9], len[9];
 };
-__device__ __forceinline__ uint32_t load_cols(Cols& cl, const Cell& q,
-                                              const uint32_t* __restrict__ cs,
+__device__ __forceinline__ uint32_t load_cols(Cols& cl, const Cell& q, const CellStarts& t,
                                               const SceneGeo& g) {
-  uint32_t hi[9];
+  uint32_t hi[9], col[9];
   bool in[9];
   const int z0 = q.z > 0 ? q.z - 1 : 0;
   const int z1 = q.z + 1 < g.dz ? q.z + 1 : g.dz - 1;
+  const int nz = z1 - z0;  // 2, at the grid's ends 1 or 0
 #pragma unroll
   for (int k = 0; k < 9; ++k) {
     const int X = q.x + k / 3 - 1;
     const int Y = q.y + k % 3 - 1;
     in[k] = (X >= 0) & (X < g.dx) & (Y >= 0) & (Y < g.dy);
-    const uint32_t col = g.base + (in[k] ? (uint32_t)((X * g.dy + Y) * g.dz) : 0u);
-    cl.lo[k] = cs[col + z0];
-    hi[k] = cs[col + z1 + 1];
+    col[k] = g.base + (in[k] ? (uint32_t)((X * g.dy + Y) * g.dz) : 0u);
+  }
+  if (t.apart) {
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      cl.lo[k] = t.cs[col[k] + z0];
+      hi[k] = t.cs[col[k] + z1 + 1];
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+      // entries z0 .. z0 + 3 (past the table's end: zeros, not used)
+      const pbf_i32x4 e =
+          pbf_raw_buffer_load_i32x4(t.buf.r, (int)((col[k] + (uint32_t)z0) << 2), 0, 0);
+      cl.lo[k] = (uint32_t)e.x;
+      hi[k] = (uint32_t)(nz == 2 ? e.w : (nz == 1 ? e.z : e.y));
+    }
   }
   uint32_t m = 0;
 #pragma unroll
@@ -310,10 +347,9 @@ __device__ __forceinline__ uint32_t write_seq(const SeqTable& st, const Cols& cl
 }
 
 __device__ __forceinline__ uint32_t build_seq(const SeqTable& st, const Cell& q,
-                                              const uint32_t* __restrict__ cs,
-                                              const SceneGeo& g) {
+                                              const CellStarts& starts, const SceneGeo& g) {
   Cols cl;
-  load_cols(cl, q, cs, g);
+  load_cols(cl, q, starts, g);
   return write_seq(st, cl, [](int, uint32_t lo) { return lo; });
 }
 
@@ -376,26 +412,57 @@ struct SeqCursor {
     while (u >= n0) shift();
     return b0 + (u - c0);
   }
-  // Byte offsets (16-byte elements) of positions p0 .. p0+7: off[t] - 16 t
-  // is the offset of the current column's element for t < n0 - p0 and of
+  // Byte offsets (elements of 2^kShift bytes) of positions p0 .. p0+7: off[t] -
+  // (t << kShift) is the offset of the current column's element for t < n0 - p0 and of
   // the next column's beyond, so each position costs one select.
   // Positions past the batch's last valid one get offsets the caller's
   // valid-bit mask discards: at most 7 elements past the end of the last
   // column or of the sequence's slot range (see load_next).  A batch
   // spanning more than two columns takes the per-position slot walk.
+  template <int kShift>
   __device__ __forceinline__ void offsets8(uint32_t p0, uint32_t last_valid, uint32_t off[8]) {
     const uint32_t last = p0 + 7u < last_valid ? p0 + 7u : last_valid;
     if (last < n1) {
       const uint32_t s = n0 - p0;  // positions of the current column in the batch
-      const uint32_t oa = (b0 + (p0 - c0)) << 4;
-      const uint32_t ob = (b1 + p0 - n0) << 4;  // wraps for t < s: not selected
+      const uint32_t oa = (b0 + (p0 - c0)) << kShift;
+      const uint32_t ob = (b1 + p0 - n0) << kShift;  // wraps for t < s: not selected
 #pragma unroll
-      for (int t = 0; t < 8; ++t) off[t] = ((uint32_t)t < s ? oa : ob) + 16u * (uint32_t)t;
+      for (int t = 0; t < 8; ++t) off[t] = ((uint32_t)t < s ? oa : ob) + ((uint32_t)t << kShift);
       if (last >= n0) shift();
     } else {
 #pragma unroll
-      for (int t = 0; t < 8; ++t) off[t] = slot(p0 + t < last_valid ? p0 + t : last_valid) << 4;
+      for (int t = 0; t < 8; ++t) off[t] = slot(p0 + t < last_valid ? p0 + t : last_valid) << kShift;
     }
+  }
+  // The same for 8-byte elements loaded in pairs: pair k (positions p0 + 2k and
+  // the next) at byte offset pair[k], whose second element is the right one
+  // unless a column begins there.  In a batch of at most two columns (true)
+  // that can be one position, alone = p0 + split, at `odd[0]`, if split is odd
+  // (8: none); in any other (false) the second elements are at odd[k].
+  __device__ __forceinline__ bool pairs8(uint32_t p0, uint32_t last_valid, uint32_t pair[4],
+                                         uint32_t odd[4], uint32_t& split) {
+    const uint32_t last = p0 + 7u < last_valid ? p0 + 7u : last_valid;
+    if (last < n1) {
+      const uint32_t s = n0 - p0;  // positions of the current column in the batch
+      const uint32_t oa = (b0 + (p0 - c0)) << 3;
+      const uint32_t ob = (b1 + p0 - n0) << 3;  // wraps below position s: not used there
+#pragma unroll
+      for (int k = 0; k < 4; ++k) pair[k] = (2u * (uint32_t)k < s ? oa : ob) + 16u * (uint32_t)k;
+      odd[0] = ob + 8u * s;
+      split = s < 8u && (s & 1u) ? s : 8u;
+      if (last >= n0) shift();
+      return true;
+    }
+    uint32_t off[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) off[t] = slot(p0 + t < last_valid ? p0 + t : last_valid) << 3;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      pair[k] = off[2 * k];
+      odd[k] = off[2 * k + 1];
+    }
+    split = 8u;
+    return false;
   }
 };
 
@@ -423,22 +490,16 @@ struct SeqCursor1 {
 };
 
 // The hit mask of the candidates [bb, be) (at most 64, one canonical block)
-// of a target's sequence as two 32-bit words: eight screening loads in flight
-// at a time; test8 turns their eight elements into eight bits.  c1 walks forward only.
-template <class LoadS, class Test8>
+// of a target's sequence as two 32-bit words: sc.batch() screens eight at a
+// time, their loads in flight together.  c1 walks forward only.
+template <class Screen>
 __device__ __forceinline__ void screen_block(SeqCursor& c1, uint32_t bb, uint32_t be,
-                                             LoadS&& load_s, Test8&& test8, uint32_t& lo,
-                                             uint32_t& hi) {
+                                             const Screen& sc, uint32_t& lo, uint32_t& hi) {
   lo = hi = 0u;
 #pragma unroll 1
   for (uint32_t u = bb; u < be; u += 8) {
-    uint32_t off[8];
-    c1.offsets8(u, be - 1u, off);
-    float3 d[8];
-#pragma unroll
-    for (int t = 0; t < 8; ++t) d[t] = load_s(off[t]);
     const uint32_t valid = be - u >= 8u ? 0xFFu : (1u << (be - u)) - 1u;
-    const uint32_t bits = test8(d) & valid;
+    const uint32_t bits = sc.batch(c1, u, be - 1u) & valid;
     const uint32_t at = u - bb;  // the same for every lane
     if (at < 32u)
       lo |= bits << at;
@@ -448,9 +509,9 @@ __device__ __forceinline__ void screen_block(SeqCursor& c1, uint32_t bb, uint32_
 }
 
 // Visits sequence positions [u0, u1) of a candidate sequence of m positions
-// in order, calling add() only for candidates passing the cheap test8 on their
-// x, y, z (load_s(byte offset of the slot's 16-byte element)).  The
-// positions are taken in groups of NB blocks of 64: each block of the group
+// in order, calling add() only for candidates passing the screen's test (see
+// ScreenXyz, ScreenCoarse).  The positions are taken in groups of NB blocks of
+// 64: each block of the group
 // is screened eight loads at a time (across column boundaries, so a sparse
 // neighbourhood costs a few memory round trips, not one or two per column)
 // into a hit mask, then the hits of the whole group are reloaded G at a time
@@ -472,12 +533,12 @@ __device__ __forceinline__ void screen_block(SeqCursor& c1, uint32_t bb, uint32_
 // get_mask(b, lo, hi) may supply block b's hit mask (b = position / 64; u0
 // must be a multiple of 64) instead of screening it; put_mask(b, lo, hi)
 // receives each mask the sweep screened.
-template <int G, int NB, class LoadS, class LoadF, class Test8, class Add, class BlockEnd,
-          class GetMask, class PutMask>
+template <int G, int NB, class Screen, class LoadF, class Add, class BlockEnd, class GetMask,
+          class PutMask>
 __device__ __forceinline__ void sweep_seq(const SeqTable& st, uint32_t m, uint32_t u0,
-                                          uint32_t u1, LoadS&& load_s, LoadF&& load_f,
-                                          Test8&& test8, Add&& add, BlockEnd&& block_end,
-                                          GetMask&& get_mask, PutMask&& put_mask) {
+                                          uint32_t u1, const Screen& sc, LoadF&& load_f,
+                                          Add&& add, BlockEnd&& block_end, GetMask&& get_mask,
+                                          PutMask&& put_mask) {
   if (u0 >= u1) return;
   constexpr int NW = 2 * NB;
   SeqCursor c1;
@@ -493,7 +554,7 @@ __device__ __forceinline__ void sweep_seq(const SeqTable& st, uint32_t m, uint32
       w[2 * q] = w[2 * q + 1] = 0u;
       if (bb < u1 && !get_mask(bb >> 6, w[2 * q], w[2 * q + 1])) {
         const uint32_t be = u1 - bb < 64u ? u1 : bb + 64u;
-        screen_block(c1, bb, be, load_s, test8, w[2 * q], w[2 * q + 1]);
+        screen_block(c1, bb, be, sc, w[2 * q], w[2 * q + 1]);
         put_mask(bb >> 6, w[2 * q], w[2 * q + 1]);
       }
     }
@@ -568,6 +629,9 @@ struct HeavyLists {
   float* partials;     // per partial slot the pass's running sum, packed (at most
                        // kPartialWords floats)
   uint32_t item_cap;   // capacity of items / partials
+  // screening coordinates of the positions the pass screens, for the policies
+  // that use them (kCoarse), in the order of screen()
+  uint2* coarse;
   // hit masks of the current iteration: block b of target i at
   // masks[b * mask_stride + i], b < kMaskBlocks (null: not kept)
   uint64_t* masks;

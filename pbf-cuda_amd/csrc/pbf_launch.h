@@ -72,17 +72,22 @@ void launch_count_place(const uint32_t* key, const uint32_t* arrival, uint2* lis
 // receive the sorted keys and their input indices.
 void launch_place_ranked(int layout, const uint32_t* key, const uint32_t* arrival, uint2* list,
                          const float* pos, const float4* xp, const uint32_t* iid, int n,
-                         long long cells, uint32_t* tile_sum, uint32_t* cs, float4* x0s,
-                         float4* xa, uint32_t* iid_s, uint32_t* cnt, uint32_t* skey,
-                         uint32_t* sval, hipStream_t st);
+                         const StepConsts& c, uint32_t* tile_sum, uint32_t* cs, float4* x0s,
+                         float4* xa, uint2* coarse, uint32_t* iid_s, uint32_t* cnt,
+                         uint32_t* skey, uint32_t* sval, hipStream_t st);
+// Where the screening coordinates of a pass of n particles go (null: it screens
+// positions); coarse below and above: the place for those of xa, or null.
+uint2* coarse_of(const HeavyLists& hl, int n, const Shapes& sh);
 // The payload gathers after the sort also count the particles per cell from
 // the sorted keys skey into cnt (all zero beforehand), the input of
 // launch_cell_starts.
 void launch_permute(int layout, const uint32_t* skey, const uint32_t* sval, const float* pos,
-                    const float4* xp, const uint32_t* iid, int n, float4* x0s, float4* xa,
-                    uint32_t* iid_s, uint32_t* cnt, hipStream_t st);
+                    const float4* xp, const uint32_t* iid, int n, const StepConsts& c,
+                    float4* x0s, float4* xa, uint2* coarse, uint32_t* iid_s, uint32_t* cnt,
+                    hipStream_t st);
 void launch_permute_pos(const uint32_t* skey, const uint32_t* sval, const float4* xp, int n,
-                        float4* xa, uint32_t* cnt, hipStream_t st);
+                        const StepConsts& c, float4* xa, uint2* coarse, uint32_t* cnt,
+                        hipStream_t st);
 // rho (may be null) receives the densities; sd and dp (null outside a tape)
 // receive (sum of lambda gradients, denominator) and the correction / pho0
 // before the clamps, per particle.

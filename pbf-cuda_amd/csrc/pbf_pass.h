@@ -6,6 +6,8 @@
 //   Target, Acc          a target's own data; its running sum (<= 8 floats)
 //   target(a, i, c)      load target i
 //   screen(a)            the float4 array whose x, y, z the screening tests
+//   kCoarse              screen on the screening coordinates (HeavyLists::coarse)
+//                        instead: every pair beyond h adds exactly 0
 //   load_f(a, j)         candidate data for the pair term
 //   hit(t, d, c)         cheap test on the candidate's x, y, z d: false only
 //                        if the pair adds exactly 0 (i itself has d == t.x)
@@ -96,6 +98,124 @@ struct MaskIO {
   }
 };
 
+// The screening test of one target for sweep_seq, eight candidates at a time.
+// ScreenXyz: positions, by the policy's near() (sign bits, one shift of a bit
+// pair each) or hit().
+template <class P, class = void>
+struct NearMode {
+  static constexpr bool value = false;
+};
+template <class P>
+struct NearMode<P, std::void_t<decltype(P::kNear)>> {
+  static constexpr bool value = P::kNear;
+};
+template <class P>
+struct ScreenXyz {
+  const Float4Buf& buf;
+  const typename P::Target& t;
+  const StepConsts& c;
+  // bits of positions u .. u + 7 (those past `last` are the caller's to mask)
+  __device__ __forceinline__ uint32_t batch(SeqCursor& c1, uint32_t u, uint32_t last) const {
+    uint32_t off[8];
+    c1.template offsets8<4>(u, last, off);
+    float3 d[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) d[k] = load_xyz_at(buf, off[k]);
+    uint32_t b = 0u;
+    if constexpr (NearMode<P>::value) {
+#pragma unroll
+      for (int k = 7; k >= 0; --k)
+        b = __builtin_amdgcn_alignbit(b, __float_as_uint(P::near(t, d[k], c)), 31u);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) b |= (P::hit(t, d[k], c) ? 1u : 0u) << k;
+    }
+    return b;
+  }
+};
+// ScreenCoarse (policies with kCoarse, whose pairs beyond h add nothing):
+// screening coordinates, singly (light kernels) or two neighbours a load (chunk
+// kernels).  A wavefront's candidates lie in ~35 cache lines however small the
+// elements are, and a load costs the L1 that many accesses, so pairs halve the
+// accesses: four loads for eight candidates, and one for a pair that two
+// columns share, or four where a batch spans more of them.  The instructions
+// for those cases cost the light kernels, whose sparse targets meet them in
+// every batch, what the accesses save.
+template <bool kPairs>
+struct ScreenCoarse {
+  const Float4Buf& buf;
+  uint2 t;
+  __device__ __forceinline__ uint32_t shift_in(uint32_t b, int xy, int z) const {
+    return __builtin_amdgcn_alignbit(
+        b, (uint32_t)screen_near(t, make_uint2((uint32_t)xy, (uint32_t)z)), 31u);
+  }
+  __device__ __forceinline__ uint32_t batch(SeqCursor& c1, uint32_t u, uint32_t last) const {
+    uint32_t b = 0u;
+    if constexpr (!kPairs) {
+      uint32_t off[8];
+      c1.template offsets8<3>(u, last, off);
+      pbf_i32x2 d[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) d[k] = pbf_raw_buffer_load_i32x2(buf.r, (int)off[k], 0, 0);
+#pragma unroll
+      for (int k = 7; k >= 0; --k) b = shift_in(b, d[k].x, d[k].y);
+    } else {
+      uint32_t pair[4], odd[4], split;
+      const bool two = c1.pairs8(u, last, pair, odd, split);
+      pbf_i32x4 d[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) d[k] = pbf_raw_buffer_load_i32x4(buf.r, (int)pair[k], 0, 0);
+      pbf_i32x2 e[4];
+      if (!two) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) e[k] = pbf_raw_buffer_load_i32x2(buf.r, (int)odd[k], 0, 0);
+      } else if (split < 8u) {
+        e[0] = pbf_raw_buffer_load_i32x2(buf.r, (int)odd[0], 0, 0);
+      }
+#pragma unroll
+      for (int k = 3; k >= 0; --k) {
+        b = shift_in(b, d[k].z, d[k].w);
+        b = shift_in(b, d[k].x, d[k].y);
+      }
+      if (!two) {
+        uint32_t o = 0u;
+#pragma unroll
+        for (int k = 3; k >= 0; --k) o = shift_in(o, e[k].x, e[k].y) << 1;
+        b = (b & 0x55u) | (o & 0xAAu);
+      } else if (split < 8u) {
+        b = (b & ~(1u << split)) | (shift_in(0u, e[0].x, e[0].y) << split);
+      }
+    }
+    return b;
+  }
+};
+template <class P, class = void>
+struct CoarseMode {
+  static constexpr bool value = false;
+};
+template <class P>
+struct CoarseMode<P, std::void_t<decltype(P::kCoarse)>> {
+  static constexpr bool value = P::kCoarse;
+};
+// The array a pass screens (kC: its screening coordinates), and the screen of
+// target ti.
+template <class P, bool kC>
+__device__ __forceinline__ Float4Buf screen_buf(const typename P::Args& a, const HeavyLists& hl,
+                                                uint32_t n) {
+  if constexpr (kC)
+    return raw_buf(hl.coarse, (uint64_t)n * 8u);
+  else
+    return float4_buf(P::screen(a), n);
+}
+template <class P, bool kC, bool kPairs>
+__device__ __forceinline__ auto screen_of(const Float4Buf& buf, const HeavyLists& hl, uint32_t ti,
+                                          const typename P::Target& t, const StepConsts& c) {
+  if constexpr (kC)
+    return ScreenCoarse<kPairs>{buf, hl.coarse[ti]};
+  else
+    return ScreenXyz<P>{buf, t, c};
+}
+
 // Generic neighbour-pass kernels over a pass policy.
 // ---------------------------------------------------------------------------
 
@@ -108,7 +228,7 @@ struct MaskIO {
 // counters for the next pass (their previous users finished earlier on the
 // stream).  If the chunk list is full the lane sums its target itself, still
 // chunk by chunk, so the canonical order holds either way.
-template <class P, class S>
+template <class P, class S, bool kC>
 __global__ __launch_bounds__(kBlock, PBF_PASS_WAVES) void k_light(typename P::Args a, int n,
                                                                   StepConsts c, S sc,
                                                                   const uint32_t* __restrict__ cs,
@@ -135,12 +255,13 @@ __global__ __launch_bounds__(kBlock, PBF_PASS_WAVES) void k_light(typename P::Ar
   const int i = block_base + tid;
   const bool active = i < n;
   const SeqTable st{&seq_dyn[tid], nb};
+  const CellStarts starts = cell_starts(cs, c.cells, n);
   typename P::Target t{};
   uint32_t m = 0;
   if (active) {
     t = P::target(a, (uint32_t)i, c);
     const SceneGeo g = sc.at((uint32_t)i, c);
-    m = build_seq(st, cell_of(t.x.x, t.x.y, t.x.z, g, c.h), cs, g);
+    m = build_seq(st, cell_of(t.x.x, t.x.y, t.x.z, g, c.h), starts, g);
   }
   {
     // this pass's statistics for the next pass's threshold: per level, how
@@ -252,7 +373,6 @@ __global__ __launch_bounds__(kBlock, PBF_PASS_WAVES) void k_light(typename P::Ar
   const uint32_t ti = (uint32_t)(block_base + src);
   const SeqTable sts{&seq_dyn[src], nb};
   t = P::target(a, ti, c);
-  auto test8 = [&](const float3 (&d)[8]) { return Test8<P, typename P::Target>::bits(t, d, c); };
   // the sweep's blocks are the canonical chunks: each is summed from zero
   // and added to the total in order (also for a heavy target whose chunk
   // list was full)
@@ -265,21 +385,21 @@ __global__ __launch_bounds__(kBlock, PBF_PASS_WAVES) void k_light(typename P::Ar
   };
   auto get_mask = [&](uint32_t b, uint32_t& lo, uint32_t& hi) { return mio.get(b, lo, hi); };
   auto put_mask = [&](uint32_t b, uint32_t lo, uint32_t hi) { mio.put(b, lo, hi); };
-  const Float4Buf sb = float4_buf(P::screen(a), (uint32_t)n);
+  const Float4Buf sb = screen_buf<P, kC>(a, hl, (uint32_t)n);
   // a pass on stored hit masks screens nothing: its hits of up to four
   // blocks run through one loop (kLightMax candidates), which balances the
   // lanes best
   constexpr int kGroup = MaskMode<P>::value == kMaskLoad ? (int)(kLightMax / kChunk) : kLightGroup;
   sweep_seq<P::kHitBatch, kGroup>(
-      sts, ms, 0u, ms, [&](uint32_t off) { return load_xyz_at(sb, off); },
-      [&](uint32_t j) { return P::load_f(a, j); }, test8, add, block_end, get_mask, put_mask);
+      sts, ms, 0u, ms, screen_of<P, kC, false>(sb, hl, ti, t, c),
+      [&](uint32_t j) { return P::load_f(a, j); }, add, block_end, get_mask, put_mask);
   P::finish(a, t, s, c, sc.at(ti, c));
 }
 
 // One work-item per chunk item (i, chunk, partial slot): the partial sum of
 // kChunk consecutive candidates of a heavy target.  Grid-stride over the
 // items; the grid size is a launch shape.
-template <class P, class S>
+template <class P, class S, bool kC>
 __global__ __launch_bounds__(kBlock, PBF_PASS_WAVES) void k_chunks(typename P::Args a, int n,
                                                                    StepConsts c, S sc,
                                                    const uint32_t* __restrict__ cs, HeavyLists hl,
@@ -296,21 +416,21 @@ __global__ __launch_bounds__(kBlock, PBF_PASS_WAVES) void k_chunks(typename P::A
       P::kXcdRanges ? xcd_runs<kChunkRun>((int)blockIdx.x, active) : (int)blockIdx.x;
   const uint32_t stride = (uint32_t)active * kBlock;
   const SeqTable st{&seq[0][threadIdx.x], kBlock};
-  const Float4Buf sb = float4_buf(P::screen(a), (uint32_t)n);
+  const CellStarts starts = cell_starts(cs, c.cells, n);
+  const Float4Buf sb = screen_buf<P, kC>(a, hl, (uint32_t)n);
   for (uint32_t u = (uint32_t)vb * kBlock + threadIdx.x; u < total; u += stride) {
     const uint4 it = hl.items[u];
     if (it.x == ~0u) continue;
     const typename P::Target t = P::target(a, it.x, c);
     const SceneGeo g = sc.at(it.x, c);
-    const uint32_t m = build_seq(st, cell_of(t.x.x, t.x.y, t.x.z, g, c.h), cs, g);
+    const uint32_t m = build_seq(st, cell_of(t.x.x, t.x.y, t.x.z, g, c.h), starts, g);
     typename P::Acc part;
     const uint32_t s0 = it.y * kChunk;
     const uint32_t s1 = s0 + kChunk < m ? s0 + kChunk : m;
     const MaskIO<P> mio{hl, it.x, m};
     sweep_seq<P::kHitBatch, 1>(
-        st, m, s0, s1, [&](uint32_t off) { return load_xyz_at(sb, off); },
+        st, m, s0, s1, screen_of<P, kC, true>(sb, hl, it.x, t, c),
         [&](uint32_t j) { return P::load_f(a, j); },
-        [&](const float3 (&d)[8]) { return Test8<P, typename P::Target>::bits(t, d, c); },
         [&](uint32_t j, const auto& d) { P::add(part, t, j, d, c, a); }, [] {},
         [&](uint32_t b, uint32_t& lo, uint32_t& hi) { return mio.get(b, lo, hi); },
         [&](uint32_t b, uint32_t lo, uint32_t hi) { mio.put(b, lo, hi); });
@@ -400,6 +520,31 @@ inline int team_blocks(int n, int lanes) {
   return (n + targets - 1) / targets;
 }
 
+// Whether a pass of n particles screens on the screening coordinates (if its
+// policy can).  From about a million particles on the L1's accesses bound the
+// chunk kernels and every load the light kernels: 1M dense step 2264 -> 2150 us,
+// 4M sweeping-wall frame 15.65 -> 14.48 ms, 64 scenes 8.69 -> 8.25 ms.  Smaller
+// passes wait on latency, and the hits' reloads no longer find the lines that
+// screening positions brought: 128K 393 / 824 / 863 -> 409 / 846 / 894 us (fresh
+// lattice / dam after 20 and 50 frames), 512K 785 / 1216 / 1040 -> 805 / 1189 /
+// 1058.
+constexpr int kCoarseMin = (1 << 19) + 1;
+inline bool coarse_screen(int n, const Shapes& sh) {
+  return n >= kCoarseMin && team_lanes(n, sh) == 0;
+}
+
+template <class P, class S, bool kC>
+void launch_lanes(const typename P::Args& a, int n, const StepConsts& c, const S& sc,
+                  const uint32_t* cs, const HeavyLists& hl, int pass, const Shapes& sh,
+                  hipStream_t st) {
+  const int lb = sh.light_block;
+  k_light<P, S, kC><<<(n + lb - 1) / lb, lb, light_lds_bytes(lb), st>>>(
+      a, n, c, sc, cs, hl, pass, (uint32_t)sh.heavy);
+  k_chunks<P, S, kC><<<grid_for_items(hl.item_cap, sh.chunk_blocks), kBlock, 0, st>>>(
+      a, n, c, sc, cs, hl, pass);
+  k_combine<P, S><<<grid_for_items(n, 512), kBlock, 0, st>>>(a, n, c, sc, hl, pass);
+}
+
 template <class P, class S>
 void launch_pass_s(const typename P::Args& a, int n, const StepConsts& c, const S& sc,
                    const uint32_t* cs, const HeavyLists& hl, int pass, const Shapes& sh,
@@ -413,12 +558,13 @@ void launch_pass_s(const typename P::Args& a, int n, const StepConsts& c, const 
     k_team<P, S, 8><<<team_blocks(n, 8), kTeamBlock, 0, st>>>(a, n, c, sc, cs);
     return;
   }
-  const int lb = sh.light_block;
-  k_light<P, S><<<(n + lb - 1) / lb, lb, light_lds_bytes(lb), st>>>(
-      a, n, c, sc, cs, hl, pass, (uint32_t)sh.heavy);
-  k_chunks<P, S><<<grid_for_items(hl.item_cap, sh.chunk_blocks), kBlock, 0, st>>>(a, n, c, sc,
-                                                                                    cs, hl, pass);
-  k_combine<P, S><<<grid_for_items(n, 512), kBlock, 0, st>>>(a, n, c, sc, hl, pass);
+  if constexpr (CoarseMode<P>::value) {
+    if (coarse_screen(n, sh)) {
+      launch_lanes<P, S, true>(a, n, c, sc, cs, hl, pass, sh, st);
+      return;
+    }
+  }
+  launch_lanes<P, S, false>(a, n, c, sc, cs, hl, pass, sh, st);
 }
 
 template <class P>

@@ -35,6 +35,7 @@ namespace {
 struct LambdaPass {
   static constexpr bool kXcdRanges = true;  // one contiguous range per XCD
   static constexpr int kMask = kMaskStore;  // hit masks for the delta-p pass
+  static constexpr bool kCoarse = true;
   // hits reloaded per round of the sweep
   static constexpr int kHitBatch = 4;
   struct Args {
@@ -152,6 +153,7 @@ struct DeltaPass {
     const float4* __restrict__ xl;
     float4* __restrict__ xa;
     float4* __restrict__ dp;  // tape only (else null): the correction / pho0 before clamps
+    uint2* __restrict__ coarse;  // screening coordinates of xa (null: not used)
   };
   struct Target {
     float4 x;  // w = lambda_i
@@ -233,6 +235,7 @@ struct DeltaPass {
     const float y = fmaxf(fminf(t.x.y + py, g.hiy), g.loy);
     const float z = fmaxf(fminf(t.x.z + pz, g.hiz), g.loz);
     a.xa[t.i] = make_float4(x, y, z, 0.0f);
+    if (a.coarse) a.coarse[t.i] = screen_coords(x, y, z, c);
     return make_float3(x, y, z);
   }
   static __device__ __forceinline__ void finish(const Args& a, const Target& t, const Acc& s,
@@ -279,6 +282,7 @@ struct DeltaLastPass : DeltaPass {
 template <int L>
 struct XsphPass {
   static constexpr bool kXcdRanges = true;  // one contiguous range per XCD
+  static constexpr bool kCoarse = true;
   // hits reloaded per round of the sweep
   static constexpr int kHitBatch = 4;
   struct Args {
@@ -366,6 +370,7 @@ struct XsphPass {
 // error statistic: |rho/pho0 - 1| per particle in FP64.
 struct DensityPass {
   static constexpr bool kXcdRanges = true;  // one contiguous range per XCD
+  static constexpr bool kCoarse = true;
   // hits reloaded per round of the sweep
   static constexpr int kHitBatch = 4;
   struct Args {
@@ -658,28 +663,34 @@ template <int L>
 __global__ __launch_bounds__(kBlock) void k_permute(
     const uint32_t* __restrict__ skey, const uint32_t* __restrict__ sval,
     const float* __restrict__ pos, const float4* __restrict__ xp,
-    const uint32_t* __restrict__ iid, int n, float4* __restrict__ x0s,
-    float4* __restrict__ xa, uint32_t* __restrict__ iid_s, uint32_t* __restrict__ cnt) {
+    const uint32_t* __restrict__ iid, int n, StepConsts c, float4* __restrict__ x0s,
+    float4* __restrict__ xa, uint2* __restrict__ coarse, uint32_t* __restrict__ iid_s,
+    uint32_t* __restrict__ cnt) {
   const int s = blockIdx.x * kBlock + threadIdx.x;
   if (blockIdx.x * kBlock >= n) return;  // whole workgroup past the end
   count_sorted(skey, s, n, cnt);
   if (s >= n) return;
   const uint32_t src = sval[s] < (uint32_t)n ? sval[s] : 0u;
   x0s[s] = load_vec<L>(pos, src);
-  xa[s] = xp[src];
+  const float4 x = xp[src];
+  xa[s] = x;
+  if (coarse) coarse[s] = screen_coords(x.x, x.y, x.z, c);
   iid_s[s] = iid[src];
 }
 
 __global__ __launch_bounds__(kBlock) void k_permute_pos(const uint32_t* __restrict__ skey,
                                                         const uint32_t* __restrict__ sval,
                                                         const float4* __restrict__ xp, int n,
-                                                        float4* __restrict__ xa,
+                                                        StepConsts c, float4* __restrict__ xa,
+                                                        uint2* __restrict__ coarse,
                                                         uint32_t* __restrict__ cnt) {
   const int s = blockIdx.x * kBlock + threadIdx.x;
   if (blockIdx.x * kBlock >= n) return;
   count_sorted(skey, s, n, cnt);
   if (s >= n) return;
-  xa[s] = xp[sval[s] < (uint32_t)n ? sval[s] : 0u];
+  const float4 x = xp[sval[s] < (uint32_t)n ? sval[s] : 0u];
+  xa[s] = x;
+  if (coarse) coarse[s] = screen_coords(x.x, x.y, x.z, c);
 }
 
 // ---- the counted grid build ------------------------------------------------
@@ -709,9 +720,9 @@ template <int L>
 __global__ __launch_bounds__(kBlock) void k_permute_ranked(
     const uint2* __restrict__ list, const uint32_t* __restrict__ cs,
     const float* __restrict__ pos, const float4* __restrict__ xp,
-    const uint32_t* __restrict__ iid, int n, float4* __restrict__ x0s, float4* __restrict__ xa,
-    uint32_t* __restrict__ iid_s, uint32_t* __restrict__ cnt, uint32_t* __restrict__ skey,
-    uint32_t* __restrict__ sval) {
+    const uint32_t* __restrict__ iid, int n, StepConsts c, float4* __restrict__ x0s,
+    float4* __restrict__ xa, uint2* __restrict__ coarse, uint32_t* __restrict__ iid_s,
+    uint32_t* __restrict__ cnt, uint32_t* __restrict__ skey, uint32_t* __restrict__ sval) {
   const int t = blockIdx.x * kBlock + threadIdx.x;
   const bool valid = t < n;
   const uint2 e = list[valid ? t : n - 1];
@@ -729,6 +740,7 @@ __global__ __launch_bounds__(kBlock) void k_permute_ranked(
   cnt[e.y] = 0u;
   if (s >= (uint32_t)n) return;  // never, for consistent counts
   xa[s] = x;
+  if (coarse) coarse[s] = screen_coords(x.x, x.y, x.z, c);
   if constexpr (L != 0) {
     x0s[s] = p;
     iid_s[s] = id;
@@ -893,35 +905,42 @@ void launch_count_place(const uint32_t* key, const uint32_t* arrival, uint2* lis
 
 void launch_place_ranked(int layout, const uint32_t* key, const uint32_t* arrival, uint2* list,
                          const float* pos, const float4* xp, const uint32_t* iid, int n,
-                         long long cells, uint32_t* tile_sum, uint32_t* cs, float4* x0s,
-                         float4* xa, uint32_t* iid_s, uint32_t* cnt, uint32_t* skey,
-                         uint32_t* sval, hipStream_t st) {
-  launch_count_place(key, arrival, list, n, cells, tile_sum, cs, cnt, st);
+                         const StepConsts& c, uint32_t* tile_sum, uint32_t* cs, float4* x0s,
+                         float4* xa, uint2* coarse, uint32_t* iid_s, uint32_t* cnt,
+                         uint32_t* skey, uint32_t* sval, hipStream_t st) {
+  launch_count_place(key, arrival, list, n, c.cells, tile_sum, cs, cnt, st);
   if (!pos)
-    k_permute_ranked<0><<<blocks_for(n), kBlock, 0, st>>>(list, cs, nullptr, xp, nullptr, n,
-                                                          nullptr, xa, nullptr, cnt, skey, sval);
+    k_permute_ranked<0><<<blocks_for(n), kBlock, 0, st>>>(list, cs, nullptr, xp, nullptr, n, c,
+                                                          nullptr, xa, coarse, nullptr, cnt, skey,
+                                                          sval);
   else if (layout == 3)
-    k_permute_ranked<3><<<blocks_for(n), kBlock, 0, st>>>(list, cs, pos, xp, iid, n, x0s, xa,
-                                                          iid_s, cnt, skey, sval);
+    k_permute_ranked<3><<<blocks_for(n), kBlock, 0, st>>>(list, cs, pos, xp, iid, n, c, x0s, xa,
+                                                          coarse, iid_s, cnt, skey, sval);
   else
-    k_permute_ranked<4><<<blocks_for(n), kBlock, 0, st>>>(list, cs, pos, xp, iid, n, x0s, xa,
-                                                          iid_s, cnt, skey, sval);
+    k_permute_ranked<4><<<blocks_for(n), kBlock, 0, st>>>(list, cs, pos, xp, iid, n, c, x0s, xa,
+                                                          coarse, iid_s, cnt, skey, sval);
 }
 
 void launch_permute(int layout, const uint32_t* skey, const uint32_t* sval, const float* pos,
-                    const float4* xp, const uint32_t* iid, int n, float4* x0s, float4* xa,
-                    uint32_t* iid_s, uint32_t* cnt, hipStream_t st) {
+                    const float4* xp, const uint32_t* iid, int n, const StepConsts& c,
+                    float4* x0s, float4* xa, uint2* coarse, uint32_t* iid_s, uint32_t* cnt,
+                    hipStream_t st) {
   if (layout == 3)
-    k_permute<3><<<blocks_for(n), kBlock, 0, st>>>(skey, sval, pos, xp, iid, n, x0s, xa, iid_s,
-                                                   cnt);
+    k_permute<3><<<blocks_for(n), kBlock, 0, st>>>(skey, sval, pos, xp, iid, n, c, x0s, xa,
+                                                   coarse, iid_s, cnt);
   else
-    k_permute<4><<<blocks_for(n), kBlock, 0, st>>>(skey, sval, pos, xp, iid, n, x0s, xa, iid_s,
-                                                   cnt);
+    k_permute<4><<<blocks_for(n), kBlock, 0, st>>>(skey, sval, pos, xp, iid, n, c, x0s, xa,
+                                                   coarse, iid_s, cnt);
 }
 
 void launch_permute_pos(const uint32_t* skey, const uint32_t* sval, const float4* xp, int n,
-                        float4* xa, uint32_t* cnt, hipStream_t st) {
-  k_permute_pos<<<blocks_for(n), kBlock, 0, st>>>(skey, sval, xp, n, xa, cnt);
+                        const StepConsts& c, float4* xa, uint2* coarse, uint32_t* cnt,
+                        hipStream_t st) {
+  k_permute_pos<<<blocks_for(n), kBlock, 0, st>>>(skey, sval, xp, n, c, xa, coarse, cnt);
+}
+
+uint2* coarse_of(const HeavyLists& hl, int n, const Shapes& sh) {
+  return coarse_screen(n, sh) ? hl.coarse : nullptr;
 }
 
 void launch_lambda(const float4* xa, const uint32_t* cs, int n, const StepConsts& c,
@@ -933,7 +952,7 @@ void launch_lambda(const float4* xa, const uint32_t* cs, int n, const StepConsts
 void launch_delta(const float4* xl, const uint32_t* cs, int n, const StepConsts& c,
                   const Scenes& scn, float4* xa, float4* dp, const VelocityOut* vo,
                   const HeavyLists& hl, int pass, const Shapes& sh, hipStream_t st) {
-  const DeltaPass::Args base{xl, xa, dp};
+  const DeltaPass::Args base{xl, xa, dp, coarse_screen(n, sh) ? hl.coarse : nullptr};
   if (!vo) {
     launch_pass<DeltaPass>(base, n, c, scn, cs, hl, pass, sh, st);
   } else if (vo->layout == 3) {
