@@ -15,7 +15,7 @@
 // of target i (j in its candidate list cand(i)) depends on x_i and x_j; its
 // derivatives belong to both.  The stale grid makes candidate lists
 // one-sided (j in cand(i) does not imply i in cand(j)), and two modes
-// collect the terms (see the comment before within_one below):
+// collect the terms (see the comment before member_word below):
 //  * scatter: i sweeps cand(i) on the sorted grid, gathers its own terms
 //    and, where i is in cand(j), j's term about i; where it is not, i adds
 //    d(its term)/dx_j to j with float atomics into "extra" arrays that a
@@ -150,20 +150,46 @@ __device__ __forceinline__ float4 take_scattered(float4* __restrict__ ex, int i,
 //  * gather (kGather = true): targets and candidates in the order of a grid
 //    built on the pass's own positions (sorted by query cell).  A target
 //    sweeps that grid around its query cell, which holds every particle
-//    within h of it, and tests both memberships per pair from the packed
-//    (sorted cell, query cell) of each slot: its own term counts when j is
+//    within h of it, and tests both memberships per pair from each
+//    slot's sorted and query cell (member_word): its own term counts when j is
 //    its candidate, j's term about it when it is j's candidate.  Every term
 //    is gathered by the particle it belongs to, in a fixed order: no atomics.
 //    A pair within h whose query cells are two apart (possible only through
 //    rounding when |x_i - x_j| is within ~1e-6 h of h, where every term and
 //    derivative is ~0) is the only pair this sweep can miss.
 
-// Whether packed cells a and b are at most one cell apart on every axis.
-__device__ __forceinline__ bool within_one(uint32_t a, uint32_t b) {
-  const int dx = (int)(a >> 20) - (int)(b >> 20);
-  const int dy = (int)((a >> 10) & 1023u) - (int)((b >> 10) & 1023u);
-  const int dz = (int)(a & 1023u) - (int)(b & 1023u);
-  return (uint32_t)(dx + 1) <= 2u && (uint32_t)(dy + 1) <= 2u && (uint32_t)(dz + 1) <= 2u;
+// The memberships of a gather-mode pair from one word per particle.  A sweep's
+// candidate j of target t has its query cell q_j within one of q_t on each
+// axis, so with a particle's sorted cell s kept as q + clamp(s - q, +-3) both
+// tests, |s_j - q_t| <= 1 and |s_t - q_j| <= 1, hold exactly when they hold
+// modulo 8.  Six fields of 5 bits: that sorted cell's x, y, z, then q's, each
+// modulo 8 plus 9; a difference of fields then ends in (difference + 1) modulo
+// 8, which is at most 2 where the test holds.
+// The word travels in the w of an element that the pass loads anyway (the lambda pass, which
+// has none free, loads it apart).  Two packed cells of 8 bytes a particle, compared axis by
+// axis -> this: delta-p pass of 270,000 particles 108 -> 100 us, lambda pass 57 -> 53, XSPH pass
+// 97 -> 86, a stored rollout of them 3330 -> 3205, one 4M-particle sweeping-wall frame with
+// gradients 56.7 -> 55.3 ms.
+constexpr uint32_t kMemberOnes = 0x02108421u;  // 1 in each field
+__device__ __forceinline__ uint32_t member_word(uint32_t sorted, uint32_t query) {
+  uint32_t w = 0u;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const int s = (int)((sorted >> (10 * k)) & 1023u), q = (int)((query >> (10 * k)) & 1023u);
+    const int d = s - q < -3 ? -3 : (s - q > 3 ? 3 : s - q);
+    w |= ((uint32_t)(q + d) & 7u) << (5 * k) | ((uint32_t)q & 7u) << (15 + 5 * k);
+  }
+  return w + 9u * kMemberOnes;
+}
+// A target's word as member_fails() takes it: its query cell under the
+// candidates' sorted cells and the other way about, without the 9s.
+__device__ __forceinline__ uint32_t member_target(uint32_t w) {
+  const uint32_t v = w - 9u * kMemberOnes;
+  return v >> 15 | (v & 0x7fffu) << 15;
+}
+// Bits in the low 15: j is no candidate of t; above: t is none of j.
+__device__ __forceinline__ uint32_t member_fails(uint32_t target, uint32_t word) {
+  return (((word - target) & 7u * kMemberOnes) + 5u * kMemberOnes) & 8u * kMemberOnes;
 }
 
 // Memberships of a pair (target t, candidate j): own = j is a candidate of
@@ -172,14 +198,14 @@ struct Members {
   bool own, other;
 };
 template <bool kGather>
-__device__ __forceinline__ Members members(const Cell& ct, uint2 tc, const float4& xj, uint2 jc,
-                                           const StepConsts& c) {
+__device__ __forceinline__ Members members(const Cell& ct, uint32_t tc, const float4& xj,
+                                           uint32_t jc, const StepConsts& c) {
   if constexpr (kGather) {
-    // packed (sorted cell, query cell) of t and j
-    return Members{within_one(jc.x, tc.y), within_one(tc.x, jc.y)};
+    const uint32_t v = member_fails(tc, jc);
+    return Members{(v & 0x7fffu) == 0u, v < 0x8000u};
   } else {
-    // the sweep ran over t's candidates; jc.y: j's packed query cell
-    return Members{true, is_candidate_of(ct, xj, jc.y, c)};
+    // the sweep ran over t's candidates; jc: j's packed query cell
+    return Members{true, is_candidate_of(ct, xj, jc, c)};
   }
 }
 
@@ -211,7 +237,7 @@ struct BwdXsphPass {
   struct Args {
     const float4* __restrict__ x;    // final positions
     const float4* __restrict__ vr;   // (v before XSPH, rho of the last lambda pass)
-    const float4* __restrict__ gv;   // adjoint of v after XSPH
+    const float4* __restrict__ gv;   // adjoint of v after XSPH; gather: w = member_word()
     const uint32_t* __restrict__ key;  // scatter: sorted keys
     float4* __restrict__ out_x;      // gathered (dL/dx, dL/drho)
     float4* __restrict__ out_v;      // gathered dL/dv (pair terms)
@@ -219,12 +245,11 @@ struct BwdXsphPass {
     float4* __restrict__ ex_v;       // scatter: dL/dv, kScatterCopies x ex_n
     uint32_t ex_n;
     const uint32_t* __restrict__ qc;  // scatter: packed query cells of x
-    const uint2* __restrict__ cq;     // gather: packed (sorted cell, query cell)
   };
   struct Target {
     float4 x, vr, gv;
     Cell cell;
-    uint2 c;
+    uint32_t c;  // gather: member_target()
     uint32_t i;
   };
   struct Acc {
@@ -232,20 +257,19 @@ struct BwdXsphPass {
   };
   struct Nb {
     float4 x, vr, gv;
-    uint2 c;
+    uint32_t c;  // gather: member_word(), scatter: packed query cell
   };
   static __device__ __forceinline__ Target target(const Args& a, uint32_t i, const StepConsts& c) {
+    const float4 gv = a.gv[i];
     if constexpr (kGather)
-      return Target{a.x[i], a.vr[i], a.gv[i], Cell{}, a.cq[i], i};
+      return Target{a.x[i], a.vr[i], gv, Cell{}, member_target(__float_as_uint(gv.w)), i};
     else
-      return Target{a.x[i], a.vr[i], a.gv[i], cell_of_key(a.key[i], c.g), make_uint2(0u, 0u), i};
+      return Target{a.x[i], a.vr[i], gv, cell_of_key(a.key[i], c.g), 0u, i};
   }
   static __device__ __forceinline__ const float4* screen(const Args& a) { return a.x; }
   static __device__ __forceinline__ Nb load_f(const Args& a, uint32_t j) {
-    if constexpr (kGather)
-      return Nb{a.x[j], a.vr[j], a.gv[j], a.cq[j]};
-    else
-      return Nb{a.x[j], a.vr[j], a.gv[j], make_uint2(0u, a.qc[j])};
+    const float4 gv = a.gv[j];
+    return Nb{a.x[j], a.vr[j], gv, kGather ? __float_as_uint(gv.w) : a.qc[j]};
   }
   static __device__ __forceinline__ bool hit(const Target& t, const float3& xj,
                                              const StepConsts& c) {
@@ -320,18 +344,18 @@ struct BwdDeltaPass {
   static constexpr int kHitBatch = 4;
   struct Args {
     const float4* __restrict__ xl;   // (x, lambda) of the iteration
-    const float4* __restrict__ A;    // (adjoint of the correction sum (before / pho0),
-                                     //  scatter: packed query cell of xl as float bits)
+    const float4* __restrict__ A;    // (adjoint of the correction sum (before / pho0), as
+                                     //  float bits scatter: packed query cell of xl,
+                                     //  gather: member_word())
     const uint32_t* __restrict__ key;  // scatter: sorted keys
     float4* __restrict__ out;        // gathered (dL/dx, dL/dlambda)
     float4* __restrict__ ex;         // scatter: (dL/dx, dL/dlambda), kScatterCopies x ex_n
     uint32_t ex_n;
-    const uint2* __restrict__ cq;    // gather: packed (sorted cell, query cell)
   };
   struct Target {
     float4 x, A;
     Cell cell;
-    uint2 c;
+    uint32_t c;  // gather: member_target()
     uint32_t i;
   };
   struct Acc {
@@ -339,29 +363,28 @@ struct BwdDeltaPass {
   };
   struct Nb {
     float4 x, A;
-    uint2 c;
+    uint32_t c;  // gather: member_word(), scatter: packed query cell
   };
   static __device__ __forceinline__ Target target(const Args& a, uint32_t i, const StepConsts& c) {
+    const float4 A = a.A[i];
     if constexpr (kGather)
-      return Target{a.xl[i], a.A[i], Cell{}, a.cq[i], i};
+      return Target{a.xl[i], A, Cell{}, member_target(__float_as_uint(A.w)), i};
     else
-      return Target{a.xl[i], a.A[i], cell_of_key(a.key[i], c.g), make_uint2(0u, 0u), i};
+      return Target{a.xl[i], A, cell_of_key(a.key[i], c.g), 0u, i};
   }
   static __device__ __forceinline__ const float4* screen(const Args& a) { return a.xl; }
   static __device__ __forceinline__ Nb load_f(const Args& a, uint32_t j) {
-    if constexpr (kGather) {
-      return Nb{a.xl[j], a.A[j], a.cq[j]};
-    } else {
-      const float4 A = a.A[j];
-      return Nb{a.xl[j], A, make_uint2(0u, __float_as_uint(A.w))};
-    }
+    const float4 A = a.A[j];
+    return Nb{a.xl[j], A, __float_as_uint(A.w)};
   }
   static __device__ __forceinline__ bool hit(const Target& t, const float3& xj,
                                              const StepConsts& c) {
     float dx, dy, dz;
     // i itself and coincident pairs (r2 = 0) add nothing; pairs closer than
     // KERNAL_EPS add nothing here either (add() drops them) but are hits of
-    // the lambda pass, which uses these masks
+    // the lambda pass, which uses these masks.  With coincident pairs let
+    // through (near(), or the screening coordinates) the chunk items of piles
+    // take 1437 us instead of 935 (4M particles under the sweeping wall).
     const float r2 = dist2(t.x, xj, dx, dy, dz);
     return (r2 < c.h2_outer) & (r2 > 0.0f);
   }
@@ -427,14 +450,13 @@ struct BwdLambdaPass {
     float4* gout;       // gin + gathered (sorted order; may alias gin)
     float4* __restrict__ ex;         // scatter: dL/dx, kScatterCopies x ex_n
     uint32_t ex_n;
-    const uint32_t* __restrict__ qc;   // scatter: packed query cells of x
-    const uint2* __restrict__ cq;      // gather: packed (sorted cell, query cell)
+    const uint32_t* __restrict__ qc;   // scatter: packed query cells of x, gather: member_word()s
     const uint32_t* __restrict__ slot;  // gather: sorted slot of each query slot
   };
   struct Target {
     float4 x, sd;
     Cell cell;
-    uint2 c;
+    uint32_t c;  // gather: member_target()
     uint32_t i;
   };
   struct Acc {
@@ -442,20 +464,17 @@ struct BwdLambdaPass {
   };
   struct Nb {
     float4 x, sd;
-    uint2 c;
+    uint32_t c;  // gather: member_word(), scatter: packed query cell
   };
   static __device__ __forceinline__ Target target(const Args& a, uint32_t i, const StepConsts& c) {
     if constexpr (kGather)
-      return Target{a.xr[i], a.sd[i], Cell{}, a.cq[i], i};
+      return Target{a.xr[i], a.sd[i], Cell{}, member_target(a.qc[i]), i};
     else
-      return Target{a.xr[i], a.sd[i], cell_of_key(a.key[i], c.g), make_uint2(0u, 0u), i};
+      return Target{a.xr[i], a.sd[i], cell_of_key(a.key[i], c.g), 0u, i};
   }
   static __device__ __forceinline__ const float4* screen(const Args& a) { return a.xr; }
   static __device__ __forceinline__ Nb load_f(const Args& a, uint32_t j) {
-    if constexpr (kGather)
-      return Nb{a.xr[j], a.sd[j], a.cq[j]};
-    else
-      return Nb{a.xr[j], a.sd[j], make_uint2(0u, a.qc[j])};
+    return Nb{a.xr[j], a.sd[j], a.qc[j]};
   }
   static __device__ __forceinline__ bool hit(const Target& t, const float3& xj,
                                              const StepConsts& c) {
@@ -660,14 +679,15 @@ __global__ __launch_bounds__(kBlock) void k_bwd_gather_iter(
     int n, const uint32_t* __restrict__ skey, uint32_t* perm, const uint2* __restrict__ list,
     const uint32_t* __restrict__ cs, const float4* __restrict__ xl, const float4* __restrict__ A,
     const uint32_t* __restrict__ pc, float4* __restrict__ xq, float4* __restrict__ aq,
-    uint2* __restrict__ cq, uint32_t* __restrict__ cnt) {
+    uint32_t* __restrict__ mw, uint32_t* __restrict__ cnt) {
   if (blockIdx.x * kBlock >= n) return;  // whole workgroup past the end
   const QuerySlot q = query_slot(n, skey, perm, list, cs, cnt);
   if (!q.valid) return;
   const float4 a = A[q.s];
   xq[q.u] = xl[q.s];
-  aq[q.u] = a;
-  cq[q.u] = make_uint2(pc[q.s], __float_as_uint(a.w));
+  const uint32_t w = member_word(pc[q.s], __float_as_uint(a.w));
+  aq[q.u] = make_float4(a.x, a.y, a.z, __uint_as_float(w));
+  mw[q.u] = w;
 }
 
 // Gather mode: the inputs of the XSPH pass in query order.
@@ -676,8 +696,7 @@ __global__ __launch_bounds__(kBlock) void k_bwd_gather_xsph(
     const uint2* __restrict__ list, const uint32_t* __restrict__ cs,
     const float4* __restrict__ x, const float4* __restrict__ vr, const float4* __restrict__ gv,
     const uint32_t* __restrict__ pc, float4* __restrict__ xq, float4* __restrict__ vrq,
-    float4* __restrict__ gvq, uint2* __restrict__ cq, uint2* __restrict__ coarse,
-    uint32_t* __restrict__ cnt) {
+    float4* __restrict__ gvq, uint2* __restrict__ coarse, uint32_t* __restrict__ cnt) {
   if (blockIdx.x * kBlock >= n) return;  // whole workgroup past the end
   const QuerySlot q = query_slot(n, skey, perm, list, cs, cnt);
   if (!q.valid) return;
@@ -686,8 +705,8 @@ __global__ __launch_bounds__(kBlock) void k_bwd_gather_xsph(
   xq[q.u] = p;
   if (coarse) coarse[q.u] = screen_coords(p.x, p.y, p.z, c);
   vrq[q.u] = vr[q.s];
-  gvq[q.u] = gv[q.s];
-  cq[q.u] = make_uint2(pc[q.s], pack_cell(qc));
+  const float4 b = gv[q.s];
+  gvq[q.u] = make_float4(b.x, b.y, b.z, __uint_as_float(member_word(pc[q.s], pack_cell(qc))));
 }
 
 // DensityBoundary slope (fluids/Simulator.cu:139-161) at wall distance d.
@@ -921,12 +940,12 @@ void launch_bwd_xsph(const BwdFrame& f, int n, const StepConsts& c, const uint32
     const QueryOrder o = order_query(q, n, c, hl, st);
     k_bwd_gather_xsph<<<blocks_for(n), kBlock, 0, st>>>(n, c, o.skey, o.perm, o.list, q.cs,
                                                         f.x_final, f.vr, f.gv_out, q.pc, q.xq,
-                                                        q.vrq, q.gvq, q.cq,
+                                                        q.vrq, q.gvq,
                                                         coarse_of(hl, n, sh), q.cnt);
     finish_query(q, n, c, st);
     using P = BwdXsphPass<true>;
     launch_pass<P>(P::Args{q.xq, q.vrq, q.gvq, nullptr, f.out_x, f.out_v, nullptr, nullptr,
-                           (uint32_t)n, nullptr, q.cq},
+                           (uint32_t)n, nullptr},
                    n, c, Scenes{}, q.cs, hl, pass, sh, st);
     k_bwd_velocity<true><<<blocks_for(n), kBlock, 0, st>>>(n, c, o.perm, f.gx_out, f.gv_out,
                                                            f.out_x, f.out_v, nullptr, nullptr,
@@ -936,7 +955,7 @@ void launch_bwd_xsph(const BwdFrame& f, int n, const StepConsts& c, const uint32
   k_bwd_qcell<<<blocks_for(n), kBlock, 0, st>>>(n, c, f.x_final, f.qc, nullptr, nullptr, nullptr);
   using P = BwdXsphPass<false>;
   launch_pass<P>(P::Args{f.x_final, f.vr, f.gv_out, f.key, f.out_x, f.out_v, f.ex_x, f.ex_v,
-                         (uint32_t)n, f.qc, nullptr},
+                         (uint32_t)n, f.qc},
                  n, c, Scenes{}, cs, hl, pass, sh, st);
   k_bwd_velocity<false><<<blocks_for(n), kBlock, 0, st>>>(n, c, nullptr, f.gx_out, f.gv_out,
                                                           f.out_x, f.out_v, f.ex_x, f.ex_v,
@@ -953,32 +972,31 @@ void launch_bwd_iteration(const BwdFrame& f, const BwdIter& it, int last, int n,
                                                   f.r0, f.escale);
     const QueryOrder o = order_query(q, n, c, hl, st);
     k_bwd_gather_iter<<<blocks_for(n), kBlock, 0, st>>>(n, o.skey, o.perm, o.list, q.cs, it.xl,
-                                                        f.A, q.pc, q.xq, q.aq, q.cq, q.cnt);
+                                                        f.A, q.pc, q.xq, q.aq, q.mw, q.cnt);
     finish_query(q, n, c, st);
     using PD = BwdDeltaPass<true>;
-    launch_pass<PD>(PD::Args{q.xq, q.aq, nullptr, f.out_x, nullptr, (uint32_t)n, q.cq}, n, c,
+    launch_pass<PD>(PD::Args{q.xq, q.aq, nullptr, f.out_x, nullptr, (uint32_t)n}, n, c,
                     Scenes{}, q.cs, hl, pass, sh, st);
     k_bwd_lambda_pre<true><<<blocks_for(n), kBlock, 0, st>>>(n, c, last, o.perm, f.out_x,
                                                              nullptr, it.xl, it.sd, it.rho,
                                                              f.grho_x, f.gxn, q.xr, q.sdb, f.r0,
                                                              f.escale);
     using PL = BwdLambdaPass<true>;
-    launch_pass<PL>(PL::Args{q.xr, q.sdb, nullptr, f.gxn, f.gx, nullptr, (uint32_t)n, nullptr,
-                             q.cq, o.perm},
+    launch_pass<PL>(PL::Args{q.xr, q.sdb, nullptr, f.gxn, f.gx, nullptr, (uint32_t)n, q.mw,
+                             o.perm},
                     n, c, Scenes{}, q.cs, hl, pass + 1, sh, st);
     return;
   }
   k_bwd_clamp<<<blocks_for(n), kBlock, 0, st>>>(n, c, f.gx, it.xl, it.dp, f.gxn, f.A, f.qc,
                                                 nullptr, nullptr, nullptr, f.r0, f.escale);
   using PD = BwdDeltaPass<false>;
-  launch_pass<PD>(PD::Args{it.xl, f.A, f.key, f.out_x, f.ex_x, (uint32_t)n, nullptr}, n, c,
+  launch_pass<PD>(PD::Args{it.xl, f.A, f.key, f.out_x, f.ex_x, (uint32_t)n}, n, c,
                   Scenes{}, cs, hl, pass, sh, st);
   k_bwd_lambda_pre<false><<<blocks_for(n), kBlock, 0, st>>>(n, c, last, nullptr, f.out_x, f.ex_x,
                                                             it.xl, it.sd, it.rho, f.grho_x, f.gxn,
                                                             f.xr, f.sdb, f.r0, f.escale);
   using PL = BwdLambdaPass<false>;
-  launch_pass<PL>(PL::Args{f.xr, f.sdb, f.key, f.gxn, f.gxn, f.ex_x, (uint32_t)n, f.qc, nullptr,
-                           nullptr},
+  launch_pass<PL>(PL::Args{f.xr, f.sdb, f.key, f.gxn, f.gxn, f.ex_x, (uint32_t)n, f.qc, nullptr},
                   n, c, Scenes{}, cs, hl, pass + 1, sh, st);
   k_bwd_fold<<<blocks_for(n), kBlock, 0, st>>>(n, f.gxn, f.ex_x, f.gx);
 }

@@ -1703,7 +1703,7 @@ int pbf_tape_backward(pbf_solver* s, pbf_tape* t, const float* gpos, const float
     bq.aq = (float4*)(ex + v16);
     bq.xr = (float4*)(ex + 2 * v16);
     bq.sdb = (float4*)(ex + 3 * v16);
-    bq.cq = (uint2*)(ex + 4 * v16);
+    bq.mw = (uint32_t*)(ex + 4 * v16);
     bq.vrq = (float4*)ev;
     bq.gvq = (float4*)(ev + v16);
     if (s->cnt_dirty) {

@@ -22,7 +22,7 @@ struct BwdQuery {
   uint32_t* pc;                   // packed sorted cell of each sorted slot (per frame)
   float4 *xq, *aq, *xr, *sdb;     // an iteration's pass inputs in query order
   float4 *vrq, *gvq;              // the XSPH pass's inputs in query order (x in xq)
-  uint2* cq;                      // packed (sorted cell, query cell) in query order
+  uint32_t* mw;                   // an iteration's membership words in query order
 };
 
 // Scatter mode's copies of the scattered pair sums: workgroup b adds to copy b % 8 (the XCD
