@@ -75,8 +75,7 @@ __device__ __forceinline__ float poly6_slope(float t, const StepConsts& c) {
 // divides once and multiplies by the reciprocal where the forward formulas
 // divide.
 __device__ __forceinline__ float recip(float x) {
-  const float y = __builtin_amdgcn_rcpf(x);
-  return fmaf(fmaf(-x, y, 1.0f), y, y);
+  return recip_step(x, __builtin_amdgcn_rcpf(x));
 }
 
 // Hessian of k (h - r)^2 d / r (the spiky gradient with coefficient k):
@@ -394,7 +393,8 @@ struct BwdDeltaPass {
     float dx, dy, dz;
     const float r2 = dist2(t.x, nb.x, dx, dy, dz);
     if (!(r2 < c.h2_outer)) return;
-    const float r = sqrt_pair(r2);
+    const Root root = root_pair(r2);
+    const float r = root.r;
     if (!(r >= c.keps && r < c.h)) return;
     const Members mb = members<kGather>(t.cell, t.c, nb.x, nb.c, c);
     if (!(mb.own || mb.other)) return;  // no term: nothing of j may enter (0 * inf)
@@ -403,7 +403,7 @@ struct BwdDeltaPass {
     const float w = ((c.poly6 * tt) * tt) * tt;
     const float q = (t.x.w + nb.x.w) + c.coef_corr * pow_corr(w, c);
     const float ds = dscorr_dw(w, c) * poly6_slope(tt, c);  // d s_corr / dx_i is this times d
-    const SpikyHess H = spiky_hess(c.spiky, r, recip(r), c);
+    const SpikyHess H = spiky_hess(c.spiky, r, recip_step(r, root.inv), c);
     // own term A_i . (q G(d)), j's term about i -q A_j . G(d), G = phi d
     const float3 A = pair_vector(mb, t.A, nb.A);
     const float Ad = dot3(A, d);
@@ -497,10 +497,11 @@ struct BwdLambdaPass {
               poly6_slope(fmaxf(c.h2 - r2, 0.0f), c);
     float phi = 0.0f;
     float3 V = make_float3(0.0f, 0.0f, 0.0f);
-    const float r = sqrt_pair(r2);
+    const Root root = root_pair(r2);
+    const float r = root.r;
     if (r >= c.keps && r < c.h && j != t.i) {
       // gradient norms: 2 D_i H (g + S_i) + 2 D_j H (g - S_j), g = phi d
-      const SpikyHess H = spiky_hess(c.spiky_rho0, r, recip(r), c);
+      const SpikyHess H = spiky_hess(c.spiky_rho0, r, recip_step(r, root.inv), c);
       const float4 si = mb.own ? t.sd : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       const float4 sj = mb.other ? nb.sd : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
       const float ki = 2.0f * si.w;

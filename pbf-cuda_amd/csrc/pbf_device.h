@@ -722,30 +722,49 @@ __device__ __forceinline__ float3 load_xyz(const float4* __restrict__ a, uint32_
 // and no exponent is extreme: there the compiler's IEEE sequences
 // (-fhip-fp32-correctly-rounded-divide-sqrt) apply no scaling and no
 // special-case fix-up, and what remains is exactly the sequence below, so
-// the results are the IEEE results bit for bit.  sqrt_pair: the hardware
-// estimate, then the neighbour below or above it when its residual says so
-// (inputs r2 in [KERNAL_EPS^2 * 0.99, h^2 * 1.0001); a smaller input, down
-// to 0, still yields a value below KERNAL_EPS, which is all the callers
-// test).  div_pair: reciprocal estimate, one Newton step, quotient with two
-// residual corrections (numerators from 1e-18 to 1e6 over denominators from
-// KERNAL_EPS to 1e4).
-__device__ __forceinline__ float sqrt_pair(float x) {
-  const float s = __builtin_amdgcn_sqrtf(x);
-  const float dn = __int_as_float(__float_as_int(s) - 1);
-  const float up = __int_as_float(__float_as_int(s) + 1);
-  float r = fmaf(-dn, s, x) <= 0.0f ? dn : s;
-  r = fmaf(-up, s, x) > 0.0f ? up : r;
-  return r;
+// the results are the IEEE results bit for bit (tests/test_gpu_arith.py and
+// test_gpu_root.py, over all roots).  root_pair: s = x rsq(x), corrected by its
+// residual times half the estimate (inputs r2 in [KERNAL_EPS^2 * 0.99,
+// h^2 * 1.0001); a smaller input, down to 0, yields a value below KERNAL_EPS
+// or a NaN, neither of which passes the callers' r >= KERNAL_EPS).  The
+// estimate serves 1 / r as well: div_root makes its reciprocal from it by the
+// Newton step with which div_pair makes one from v_rcp_f32, then both take the
+// quotient with two residual corrections (numerators from 1e-18 to 1e6 over
+// denominators from KERNAL_EPS to 1e4).  Transcendental instructions take four
+// times as long as others: root and quotient need one and twelve others, where
+// v_sqrt_f32, corrected by its neighbours' residuals, and v_rcp_f32 needed two
+// and fifteen.  A step of 130,000 particles 604 -> 591 us, 1M dense
+// 2150 -> 2110, 64 scenes 8.24 -> 8.03 ms.
+struct Root {
+  float r, inv;  // the root; an estimate of its reciprocal
+};
+__device__ __forceinline__ Root root_pair(float x) {
+  const float y = __builtin_amdgcn_rsqf(x);
+  const float s = x * y;
+  return Root{fmaf(fmaf(-s, s, x), 0.5f * y, s), y};
 }
-__device__ __forceinline__ float div_pair(float a, float b) {
-  float r = __builtin_amdgcn_rcpf(b);
-  const float e = fmaf(-b, r, 1.0f);
-  r = fmaf(e, r, r);
+// 1 / b from an estimate within a few ulp.
+__device__ __forceinline__ float recip_step(float b, float y) {
+  return fmaf(fmaf(-b, y, 1.0f), y, y);
+}
+// The estimate a root's reciprocal starts from: one unit up.  At mantissas of
+// all ones the Newton step from v_rsq_f32's own value ends on the midpoint
+// next to 1 / b and rounds to the wrong side of it.
+__device__ __forceinline__ float root_inv(const Root& b) {
+  return __int_as_float(__float_as_int(b.inv) + 1);
+}
+__device__ __forceinline__ float div_recip(float a, float b, float r) {
   float q = a * r;
   const float rem = fmaf(-b, q, a);
   q = fmaf(rem, r, q);
   const float rem2 = fmaf(-b, q, a);
   return fmaf(rem2, r, q);
+}
+__device__ __forceinline__ float div_root(float a, const Root& b) {
+  return div_recip(a, b.r, recip_step(b.r, root_inv(b)));
+}
+__device__ __forceinline__ float div_pair(float a, float b) {
+  return div_recip(a, b, recip_step(b, __builtin_amdgcn_rcpf(b)));
 }
 
 // poly6 numerator times its coefficient, for r2 < h2: poly6 * (h2-r2)^3.

@@ -74,10 +74,11 @@ struct LambdaPass {
       if (r2 < c.h2) s.rho = s.rho + poly6_of(r2, c);
       // coincident pairs (piles clamped into a corner) have no gradient term:
       // skip their square root
-      const float r = r2 >= c.keps2_lo ? sqrt_pair(r2) : 0.0f;
+      const Root root = r2 >= c.keps2_lo ? root_pair(r2) : Root{0.0f, 0.0f};
+      const float r = root.r;
       if (r >= c.keps && r < c.h) {
         const float u = c.h - r;
-        const float f = div_pair((c.spiky_rho0 * u) * u, r);
+        const float f = div_root((c.spiky_rho0 * u) * u, root);
         const float ax = f * dx, ay = f * dy, az = f * dz;
         s.gx = s.gx + ax;
         s.gy = s.gy + ay;
@@ -100,9 +101,10 @@ struct LambdaPass {
                                               const StepConsts& c, const Args&) {
     float dx, dy, dz;
     const float r2 = dist2(t.x, xj, dx, dy, dz);
-    const float r = sqrt_pair(r2);
+    const Root root = root_pair(r2);
+    const float r = root.r;
     const float u = c.h - r;
-    const float f = div_pair((c.spiky_rho0 * u) * u, r);
+    const float f = div_root((c.spiky_rho0 * u) * u, root);
     const bool in = (r >= c.keps) & (r < c.h);
     return Term{in ? f * dx : 0.0f, in ? f * dy : 0.0f, in ? f * dz : 0.0f,
                 r2 < c.h2 ? poly6_of(r2, c) : 0.0f};
@@ -181,12 +183,13 @@ struct DeltaPass {
     float dx, dy, dz;
     const float r2 = dist2(t.x, xj, dx, dy, dz);
     if (r2 < c.h2_outer) {
-      const float r = sqrt_pair(r2);
+      const Root root = root_pair(r2);
+      const float r = root.r;
       if (r >= c.keps && r < c.h) {
         const float w = r2 < c.h2 ? poly6_of(r2, c) : 0.0f;
         const float corr = c.coef_corr * pow_corr(w, c);
         const float u = c.h - r;
-        const float gs = div_pair((c.spiky * u) * u, r);
+        const float gs = div_root((c.spiky * u) * u, root);
         const float f = ((t.x.w + xj.w) + corr) * gs;
         s.px = fmaf(f, dx, s.px);
         s.py = fmaf(f, dy, s.py);
@@ -204,11 +207,12 @@ struct DeltaPass {
                                               const StepConsts& c, const Args&) {
     float dx, dy, dz;
     const float r2 = dist2(t.x, xj, dx, dy, dz);
-    const float r = sqrt_pair(r2);
+    const Root root = root_pair(r2);
+    const float r = root.r;
     const float w = r2 < c.h2 ? poly6_of(r2, c) : 0.0f;
     const float corr = c.coef_corr * pow_corr(w, c);
     const float u = c.h - r;
-    const float gs = div_pair((c.spiky * u) * u, r);
+    const float gs = div_root((c.spiky * u) * u, root);
     const bool in = (r >= c.keps) & (r < c.h);
     return Term{in ? ((t.x.w + xj.w) + corr) * gs : 0.0f, in ? dx : 0.0f, in ? dy : 0.0f,
                 in ? dz : 0.0f};
