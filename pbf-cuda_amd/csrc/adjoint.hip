@@ -839,13 +839,12 @@ __global__ __launch_bounds__(kBlock) void k_fill_f64(double* __restrict__ a, int
   for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += stride) a[i] = 0.0;
 }
 
-// Layout conversion of a caller vector array to float4.
-template <int L>
+// A caller's vector array of layout 3 as float4.
 __global__ __launch_bounds__(kBlock) void k_to_f4(const float* __restrict__ a, int n,
                                                   float4* __restrict__ out) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
-  out[i] = load_vec<L>(a, (uint32_t)i);
+  out[i] = load_vec<3>(a, (uint32_t)i);
 }
 
 // Sum of n doubles in a fixed order (independent of the hardware's
@@ -1026,11 +1025,8 @@ void launch_fill_f64(double* a, int n, hipStream_t st) {
   k_fill_f64<<<fill_blocks(n), kBlock, 0, st>>>(a, n);
 }
 
-void launch_to_f4(int layout, const float* a, int n, float4* out, hipStream_t st) {
-  if (layout == 3)
-    k_to_f4<3><<<blocks_for(n), kBlock, 0, st>>>(a, n, out);
-  else
-    k_to_f4<4><<<blocks_for(n), kBlock, 0, st>>>(a, n, out);
+void launch_to_f4(const float* a, int n, float4* out, hipStream_t st) {
+  k_to_f4<<<blocks_for(n), kBlock, 0, st>>>(a, n, out);
 }
 
 void launch_sum_f64(const double* a, int n, double* part, double* out, hipStream_t st) {

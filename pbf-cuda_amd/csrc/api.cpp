@@ -105,7 +105,7 @@ struct GraphSig {
 // A recorded step: the launch sequence of one (arrays, n, stream)
 // combination as an instantiated HIP graph, recorded under `sig`.
 struct GraphEntry {
-  const void* key[6] = {};
+  const void* key[9] = {};
   int n = 0;
   GraphSig sig;
   hipGraph_t graph = nullptr;
@@ -417,13 +417,18 @@ void drop_graphs(pbf_solver* s) {
 
 // What a tape keeps of one frame's forward pass (all null outside a tape):
 // per iteration k the (x, lambda) array, (S, D), densities and the
-// correction before its clamps; and, set by enqueue_step, where the sorted
-// keys and the sort permutation ended up.
+// correction before its clamps; where the step keeps the grid, the positions
+// and (velocity, rho) instead of the solver's arrays (a stored tape); and, set
+// by enqueue_step, where the sorted keys and the sort permutation ended up (in
+// keep_key and keep_val, if set, from the counted grid).
 struct Record {
   float4** xl = nullptr;
   float4** sd = nullptr;
   float** rho = nullptr;
   float4** dp = nullptr;
+  uint32_t* cs = nullptr;
+  float4 *xa = nullptr, *vr = nullptr;
+  uint32_t *keep_key = nullptr, *keep_val = nullptr;
   const uint32_t* skey = nullptr;
   const uint32_t* sval = nullptr;
   // a backward pass's recompute of the frame: the XSPH pass is left out (its
@@ -432,11 +437,15 @@ struct Record {
   bool skip_xsph = false;
 };
 
-// Caller arrays of one step.
+// Caller arrays of one step.  pos, vel and iid are the step's inputs and receive
+// the sorted start positions, velocities and identities; a tape, whose inputs
+// are checkpoints, names those apart (in_*), where it would copy them otherwise.
 struct StepArrays {
   float *pos, *npos, *vel, *nvel;
   uint32_t* iid;
   int n;
+  const float *in_pos = nullptr, *in_vel = nullptr;
+  const uint32_t* in_iid = nullptr;
 };
 
 pbf::Scenes scenes_of(const pbf_solver* s) {
@@ -475,12 +484,18 @@ void enqueue_step(pbf_solver* s, const StepArrays& a, const pbf::StepConsts& c, 
   const int n = a.n;
   const pbf::Scenes scn = scenes_of(s);
   const pbf::Shapes& sh = s->shapes;
+  const float* in_pos = a.in_pos ? a.in_pos : a.pos;
+  const float* in_vel = a.in_vel ? a.in_vel : a.vel;
+  const uint32_t* in_iid = a.in_iid ? a.in_iid : a.iid;
+  uint32_t* const cs = rec && rec->cs ? rec->cs : s->cs;
+  float4* const xa = rec && rec->xa ? rec->xa : s->xa;
+  float4* const vr = rec && rec->vr ? rec->vr : s->vr;
   tb(PBF_PHASE_STEP);
   // advect() + getGridId (Simulator.cpp:50, Simulator.cu:165-193)
   const bool counted = n <= pbf::kCountedStepMax;
   uint2* const coarse = pbf::coarse_of(s->hl, n, sh);
   tb(PBF_PHASE_PREDICT);
-  pbf::launch_predict_key(L, a.pos, a.vel, n, c, scn, s->xp, s->key0, s->val0, s->counters,
+  pbf::launch_predict_key(L, in_pos, in_vel, n, c, scn, s->xp, s->key0, s->val0, s->counters,
                           counted ? s->cnt : nullptr, st);
   te(PBF_PHASE_PREDICT);
   // thrust::sort_by_key (Simulator.cu:196-198), memset + computeGridRange
@@ -488,13 +503,14 @@ void enqueue_step(pbf_solver* s, const StepArrays& a, const pbf::StepConsts& c, 
   if (counted) {
     // the work lists' records are free until the first neighbour pass
     tb(PBF_PHASE_GRID);
-    pbf::launch_place_ranked(L, s->key0, s->val0, (uint2*)s->hl.recs, a.pos, s->xp, a.iid, n, c,
-                             s->tile_sum, s->cs, s->x0s, s->xa, coarse, s->iid_s, s->cnt,
-                             rec ? s->key1 : nullptr, rec ? s->val1 : nullptr, st);
+    uint32_t* const key = rec ? (rec->keep_key ? rec->keep_key : s->key1) : nullptr;
+    uint32_t* const val = rec ? (rec->keep_val ? rec->keep_val : s->val1) : nullptr;
+    pbf::launch_place_ranked(L, s->key0, s->val0, (uint2*)s->hl.recs, in_pos, s->xp, in_iid, n, c,
+                             s->tile_sum, cs, s->x0s, xa, coarse, s->iid_s, s->cnt, key, val, st);
     te(PBF_PHASE_GRID);
     if (rec) {
-      rec->skey = s->key1;
-      rec->sval = s->val1;
+      rec->skey = key;
+      rec->sval = val;
     }
   } else {
     tb(PBF_PHASE_SORT);
@@ -510,9 +526,9 @@ void enqueue_step(pbf_solver* s, const StepArrays& a, const pbf::StepConsts& c, 
     // the payload gather counts the particles per cell, the scan turns the
     // counts into cell starts
     tb(PBF_PHASE_GRID);
-    pbf::launch_permute(L, skey, sval, a.pos, s->xp, a.iid, n, c, s->x0s, s->xa, coarse,
-                        s->iid_s, s->cnt, st);
-    pbf::launch_cell_starts(s->cnt, c.cells, s->tile_sum, s->cs, st);
+    pbf::launch_permute(L, skey, sval, in_pos, s->xp, in_iid, n, c, s->x0s, xa, coarse, s->iid_s,
+                        s->cnt, st);
+    pbf::launch_cell_starts(s->cnt, c.cells, s->tile_sum, cs, st);
     te(PBF_PHASE_GRID);
   }
   // niter x correctDensity (Simulator.cpp:62-66, Simulator.cu:213-249);
@@ -524,22 +540,22 @@ void enqueue_step(pbf_solver* s, const StepArrays& a, const pbf::StepConsts& c, 
     float4* xl = rec ? rec->xl[it] : s->xp;
     float* rho = rec ? rec->rho[it] : (it + 1 == NI ? s->rho : nullptr);
     tb(PBF_PHASE_LAMBDA);
-    pbf::launch_lambda(s->xa, s->cs, n, c, scn, xl, rho, rec ? rec->sd[it] : nullptr, s->hl,
+    pbf::launch_lambda(xa, cs, n, c, scn, xl, rho, rec ? rec->sd[it] : nullptr, s->hl,
                        pass++, sh, st);
     te(PBF_PHASE_LAMBDA);
     // the last iteration also does updateVelocity (Simulator.cpp:72,
     // Simulator.cu:267-274) as each particle's final position is known
     const pbf::VelocityOut vo{L,         s->x0s, rec ? rec->rho[NI - 1] : s->rho, s->iid_s,
-                              s->vr,     a.pos,  a.vel,                            a.iid};
+                              vr,        a.pos,  a.vel,                            a.iid};
     tb(PBF_PHASE_DELTA);
-    pbf::launch_delta(xl, s->cs, n, c, scn, s->xa, rec ? rec->dp[it] : nullptr,
+    pbf::launch_delta(xl, cs, n, c, scn, xa, rec ? rec->dp[it] : nullptr,
                       it + 1 == NI ? &vo : nullptr, s->hl, pass++, sh, st);
     te(PBF_PHASE_DELTA);
   }
   // correctVelocity (Simulator.cpp:77, Simulator.cu:251-265)
   if (!(rec && rec->skip_xsph)) {
     tb(PBF_PHASE_XSPH);
-    pbf::launch_xsph(L, s->xa, s->vr, s->cs, n, c, scn, a.npos, a.nvel, s->hl, pass, sh, st);
+    pbf::launch_xsph(L, xa, vr, cs, n, c, scn, a.npos, a.nvel, s->hl, pass, sh, st);
     te(PBF_PHASE_XSPH);
   }
   te(PBF_PHASE_STEP);
@@ -581,7 +597,8 @@ GraphSig make_sig(const pbf_solver* s, const pbf::StepConsts& c) {
 // re-instantiated if the update is refused (a different sort pass count).
 int find_or_record(pbf_solver* s, const StepArrays& a, const pbf::StepConsts& c, hipStream_t st,
                    GraphEntry** out) {
-  const void* key[6] = {a.pos, a.npos, a.vel, a.nvel, a.iid, (const void*)st};
+  const void* key[9] = {a.pos,    a.npos,   a.vel,    a.nvel, a.iid, a.in_pos,
+                        a.in_vel, a.in_iid, (const void*)st};
   const GraphSig sig = make_sig(s, c);
   for (auto& g : s->graphs) {
     if (g.n == a.n && std::memcmp(g.key, key, sizeof(key)) == 0) {
@@ -642,6 +659,49 @@ int find_or_record(pbf_solver* s, const StepArrays& a, const pbf::StepConsts& c,
   ++s->ginfo.recorded;
   ++s->ginfo.instantiated;
   *out = &s->graphs.back();
+  return PBF_OK;
+}
+
+int check_step_count(pbf_solver* s, int n) {
+  if (n > s->capacity)
+    return fail(s, PBF_ERR_CAPACITY, "n = %d exceeds capacity %d", n, s->capacity);
+  if (s->nscenes && n != s->capacity)
+    return fail(s, PBF_ERR_INVALID_ARGUMENT,
+                "a batched solver steps all its particles: n must be %d, got %d", s->capacity, n);
+  return PBF_OK;
+}
+
+// One step on arrays whose pointers have been checked: replayed from its
+// recorded graph if the solver has graphs on, else enqueued.
+int run_step(pbf_solver* s, const StepArrays& arr, void* stream) {
+  int rc;
+  pbf::StepConsts c;
+  if ((rc = step_consts(s, c))) return rc;
+  DeviceGuard g(s->device);
+  if (!g.ok) return fail(s, PBF_ERR_HIP, "hipSetDevice(%d) failed", s->device);
+  hipStream_t st = (hipStream_t)stream;
+  if (s->cnt_dirty) pbf::launch_fill_u32(s->cnt, s->max_cells, 0u, st);
+  s->cnt_dirty = true;
+  if (s->graph_on && st != nullptr) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    hipError_t e = hipStreamIsCapturing(st, &cap);
+    if (e != hipSuccess) return fail_hip(s, e, "hipStreamIsCapturing");
+    if (cap == hipStreamCaptureStatusNone) {
+      GraphEntry* ge = nullptr;
+      if ((rc = find_or_record(s, arr, c, st, &ge))) return rc;
+      tbegin(s, PBF_PHASE_STEP, st);
+      e = hipGraphLaunch(ge->exec, st);
+      tend(s, PBF_PHASE_STEP, st);
+      if (e != hipSuccess) return fail_hip(s, e, "hipGraphLaunch");
+      ++s->ginfo.replayed;
+      s->cnt_dirty = false;
+      return PBF_OK;
+    }
+  }
+  enqueue_step(s, arr, c, st, true);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail_hip(s, e, "kernel launch");
+  s->cnt_dirty = false;
   return PBF_OK;
 }
 
@@ -1019,13 +1079,9 @@ int pbf_step(pbf_solver* s, float* pos, float* npos, float* vel, float* nvel, ui
              int n, void* stream) {
   if (!s) return fail(nullptr, PBF_ERR_INVALID_ARGUMENT, "solver is NULL");
   if (n < 0) return fail(s, PBF_ERR_INVALID_ARGUMENT, "n must be >= 0, got %d", n);
-  if (n > s->capacity)
-    return fail(s, PBF_ERR_CAPACITY, "n = %d exceeds capacity %d", n, s->capacity);
-  if (s->nscenes && n != s->capacity)
-    return fail(s, PBF_ERR_INVALID_ARGUMENT,
-                "a batched solver steps all its particles: n must be %d, got %d", s->capacity, n);
-  if (n == 0) return PBF_OK;
   int rc;
+  if ((rc = check_step_count(s, n))) return rc;
+  if (n == 0) return PBF_OK;
   if ((rc = check_vec_ptr(s, pos, "pos")) || (rc = check_vec_ptr(s, npos, "npos")) ||
       (rc = check_vec_ptr(s, vel, "vel")) || (rc = check_vec_ptr(s, nvel, "nvel")))
     return rc;
@@ -1036,36 +1092,7 @@ int pbf_step(pbf_solver* s, float* pos, float* npos, float* vel, float* nvel, ui
       for (int b = a + 1; b < 5; ++b)
         if (p[a] == p[b]) return fail(s, PBF_ERR_INVALID_ARGUMENT, "particle arrays must be distinct");
   }
-  pbf::StepConsts c;
-  if ((rc = step_consts(s, c))) return rc;
-  DeviceGuard g(s->device);
-  if (!g.ok) return fail(s, PBF_ERR_HIP, "hipSetDevice(%d) failed", s->device);
-  hipStream_t st = (hipStream_t)stream;
-  const StepArrays arr{pos, npos, vel, nvel, iid, n};
-
-  if (s->cnt_dirty) pbf::launch_fill_u32(s->cnt, s->max_cells, 0u, st);
-  s->cnt_dirty = true;
-  if (s->graph_on && st != nullptr) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    hipError_t e = hipStreamIsCapturing(st, &cap);
-    if (e != hipSuccess) return fail_hip(s, e, "hipStreamIsCapturing");
-    if (cap == hipStreamCaptureStatusNone) {
-      GraphEntry* ge = nullptr;
-      if ((rc = find_or_record(s, arr, c, st, &ge))) return rc;
-      tbegin(s, PBF_PHASE_STEP, st);
-      e = hipGraphLaunch(ge->exec, st);
-      tend(s, PBF_PHASE_STEP, st);
-      if (e != hipSuccess) return fail_hip(s, e, "hipGraphLaunch");
-      ++s->ginfo.replayed;
-      s->cnt_dirty = false;
-      return PBF_OK;
-    }
-  }
-  enqueue_step(s, arr, c, st, true);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return fail_hip(s, e, "kernel launch");
-  s->cnt_dirty = false;
-  return PBF_OK;
+  return run_step(s, StepArrays{pos, npos, vel, nvel, iid, n}, stream);
 }
 
 int pbf_step_batched(pbf_solver* s, float* pos, float* npos, float* vel, float* nvel,
@@ -1581,41 +1608,42 @@ int pbf_tape_forward(pbf_solver* s, pbf_tape* t, const float* pos, const float* 
     }
     t->ul[(size_t)f] = s->ulim;
     t->ll[(size_t)f] = s->llim;
-    // the step clobbers its inputs: step a copy of checkpoint f
-    if ((e = hipMemcpyAsync(t->wpos, t->cpos[f], vb, hipMemcpyDeviceToDevice, st)) != hipSuccess ||
-        (e = hipMemcpyAsync(t->wvel, t->cvel[f], vb, hipMemcpyDeviceToDevice, st)) != hipSuccess ||
-        (e = hipMemcpyAsync(t->ciid[f + 1], t->ciid[f], ib, hipMemcpyDeviceToDevice, st)) !=
-            hipSuccess)
-      return fail_hip(s, e, "tape checkpoint copy");
+    // the step reads checkpoint f and leaves what it makes of its inputs in
+    // the work arrays.  (Copying checkpoints, stored frames and seeds instead,
+    // 26 copies of 4.4 us in a stored two-frame rollout of 270,000 particles with its
+    // gradients: 3164 us against 3112; 30 frames of 16,384 15.82 ms against
+    // 15.35.)
+    const size_t fb = (size_t)f;
+    const StepArrays arr{t->wpos,          t->cpos[fb + 1], t->wvel,     t->cvel[fb + 1],
+                         t->ciid[fb + 1],  t->n,            t->cpos[fb], t->cvel[fb],
+                         t->ciid[fb]};
     if (!t->store) {
-      if ((rc = pbf_step(s, t->wpos, t->cpos[f + 1], t->wvel, t->cvel[f + 1], t->ciid[f + 1],
-                         t->n, stream)))
-        return rc;
+      if ((rc = check_step_count(s, t->n)) || (rc = run_step(s, arr, stream))) return rc;
       continue;
     }
-    // stored tape: the step keeps its iterations in frame f's arrays, then
-    // the grid, the sort and the pre-XSPH state the adjoint reads are kept
+    // stored tape: the step keeps its iterations, the grid, the sort and the
+    // pre-XSPH state the adjoint reads in frame f's arrays
     pbf::StepConsts c;
     if ((rc = step_consts(s, c))) return rc;
-    const size_t q0 = (size_t)f * (size_t)t->niter;
+    const size_t q0 = fb * (size_t)t->niter;
     Record rec;
+    rec.cs = t->f_cs[fb];
+    rec.xa = t->f_xa[fb];
+    rec.vr = t->f_vr[fb];
+    rec.keep_key = t->f_key[fb];
+    rec.keep_val = t->f_val[fb];
     rec.xl = &t->f_xl[q0];
     rec.sd = &t->f_sd[q0];
     rec.dp = &t->f_dp[q0];
     rec.rho = &t->f_rho[q0];
     if (s->cnt_dirty) pbf::launch_fill_u32(s->cnt, s->max_cells, 0u, st);
     s->cnt_dirty = true;
-    const StepArrays arr{t->wpos, t->cpos[f + 1], t->wvel, t->cvel[f + 1], t->ciid[f + 1], t->n};
     enqueue_step(s, arr, c, st, false, &rec);
-    const size_t fb = (size_t)f, v4 = (size_t)t->n * 16;
-    if ((e = hipMemcpyAsync(t->f_key[fb], rec.skey, ib, hipMemcpyDeviceToDevice, st)) !=
-            hipSuccess ||
-        (e = hipMemcpyAsync(t->f_val[fb], rec.sval, ib, hipMemcpyDeviceToDevice, st)) !=
-            hipSuccess ||
-        (e = hipMemcpyAsync(t->f_cs[fb], s->cs, ((size_t)c.cells + 1) * 4,
-                            hipMemcpyDeviceToDevice, st)) != hipSuccess ||
-        (e = hipMemcpyAsync(t->f_xa[fb], s->xa, v4, hipMemcpyDeviceToDevice, st)) != hipSuccess ||
-        (e = hipMemcpyAsync(t->f_vr[fb], s->vr, v4, hipMemcpyDeviceToDevice, st)) != hipSuccess)
+    if (rec.skey != t->f_key[fb] &&  // the radix sort left them in the solver's arrays
+        ((e = hipMemcpyAsync(t->f_key[fb], rec.skey, ib, hipMemcpyDeviceToDevice, st)) !=
+             hipSuccess ||
+         (e = hipMemcpyAsync(t->f_val[fb], rec.sval, ib, hipMemcpyDeviceToDevice, st)) !=
+             hipSuccess))
       return fail_hip(s, e, "tape frame copy");
     if ((e = hipGetLastError()) != hipSuccess) return fail_hip(s, e, "kernel launch");
     s->cnt_dirty = false;
@@ -1651,18 +1679,20 @@ int pbf_tape_backward(pbf_solver* s, pbf_tape* t, const float* gpos, const float
       s->llim = ll;
     }
   } box_restore{s, s->ulim, s->llim};
-  const size_t vb = (size_t)n * (size_t)L * 4, ib = (size_t)n * 4;
+  const size_t vb = (size_t)n * (size_t)L * 4;
   hipError_t e;
-  // seeds: dL/d(final state), caller layout
-  if (gpos) {
-    e = hipMemcpyAsync(t->gp[0], gpos, vb, hipMemcpyDeviceToDevice, st);
-  } else {
-    e = hipMemsetAsync(t->gp[0], 0, vb, st);
+  // seeds: dL/d(final state), caller layout; read where they are unless they
+  // are rescaled in place
+  const float *gp_in = gpos, *gv_in = gvel;
+  const float* const seeds[2] = {gpos, gvel};
+  float* const seed_to[2] = {t->gp[0], t->gv[0]};
+  for (int k = 0; k < 2; ++k) {
+    if (seeds[k] && !t->rescale) continue;
+    e = seeds[k] ? hipMemcpyAsync(seed_to[k], seeds[k], vb, hipMemcpyDeviceToDevice, st)
+                 : hipMemsetAsync(seed_to[k], 0, vb, st);
+    if (e != hipSuccess) return fail_hip(s, e, "seeding the backward pass");
+    (k ? gv_in : gp_in) = seed_to[k];
   }
-  if (e == hipSuccess)
-    e = gvel ? hipMemcpyAsync(t->gv[0], gvel, vb, hipMemcpyDeviceToDevice, st)
-             : hipMemsetAsync(t->gv[0], 0, vb, st);
-  if (e != hipSuccess) return fail_hip(s, e, "seeding the backward pass");
   pbf::launch_fill_f64(t->r0, n, st);
   if (t->rescale) {
     pbf::launch_fill_u32(reinterpret_cast<uint32_t*>(t->escale), 1, 0u, st);
@@ -1755,15 +1785,11 @@ int pbf_tape_backward(pbf_solver* s, pbf_tape* t, const float* gpos, const float
       sval = t->f_val[fb];
     } else {
       // recompute frame f from its checkpoint, keeping its iterations
-      if ((e = hipMemcpyAsync(t->wpos, t->cpos[f], vb, hipMemcpyDeviceToDevice, st)) !=
-              hipSuccess ||
-          (e = hipMemcpyAsync(t->wvel, t->cvel[f], vb, hipMemcpyDeviceToDevice, st)) !=
-              hipSuccess ||
-          (e = hipMemcpyAsync(t->wiid, t->ciid[f], ib, hipMemcpyDeviceToDevice, st)) != hipSuccess)
-        return fail_hip(s, e, "tape checkpoint copy");
       if (s->cnt_dirty) pbf::launch_fill_u32(s->cnt, s->max_cells, 0u, st);
       s->cnt_dirty = true;
-      const StepArrays arr{t->wpos, t->wnpos, t->wvel, t->wnvel, t->wiid, n};
+      const size_t fb = (size_t)f;
+      const StepArrays arr{t->wpos, t->wnpos, t->wvel,      t->wnvel,   t->wiid,
+                           n,       t->cpos[fb], t->cvel[fb], t->ciid[fb]};
       enqueue_step(s, arr, c, st, false, &rec);
       for (size_t k = 0; k < (size_t)NI; ++k)
         iters[k] = pbf::BwdIter{t->xl[k], t->sd[k], t->rho[k], t->dp[k]};
@@ -1774,14 +1800,16 @@ int pbf_tape_backward(pbf_solver* s, pbf_tape* t, const float* gpos, const float
       pass = 2 * NI;
     }
     // adjoint of the frame
-    pbf::launch_to_f4(L, t->gp[cur], n, t->gxo, st);
-    pbf::launch_to_f4(L, t->gv[cur], n, t->gvo, st);
+    if (L == 3) {
+      pbf::launch_to_f4(gp_in, n, t->gxo, st);
+      pbf::launch_to_f4(gv_in, n, t->gvo, st);
+    }
     pbf::BwdFrame bf{};
     bf.x_final = x_final;
     bf.vr = vr;
     bf.key = skey;
-    bf.gx_out = t->gxo;
-    bf.gv_out = t->gvo;
+    bf.gx_out = L == 3 ? t->gxo : (const float4*)gp_in;
+    bf.gv_out = L == 3 ? t->gvo : (const float4*)gv_in;
     bf.out_x = t->out_x;
     bf.out_v = t->out_v;
     bf.ex_x = t->ex_x;
@@ -1809,6 +1837,8 @@ int pbf_tape_backward(pbf_solver* s, pbf_tape* t, const float* gpos, const float
     float* ov = f == 0 ? gvel0 : t->gv[cur ^ 1];
     pbf::launch_bwd_predict(L, bf, sval, n, c, op, ov, st);
     if (t->rescale && f > 0) pbf::launch_rescale(op, n * L, ov, n * L, t->maxbits, t->escale, st);
+    gp_in = op;
+    gv_in = ov;
     cur ^= 1;
     if ((e = hipGetLastError()) != hipSuccess) return fail_hip(s, e, "kernel launch");
     s->cnt_dirty = false;

@@ -38,7 +38,7 @@ struct BwdFrame {
   const float4* x_final;  // positions after the last iteration
   const float4* vr;       // (velocity before XSPH, rho of the last lambda pass)
   const uint32_t* key;    // sorted cell keys
-  // adjoints of the frame's outputs (read)
+  // adjoints of the frame's outputs (read; w is anything)
   const float4* gx_out;   // dL/d(final positions)
   const float4* gv_out;   // dL/d(velocities after XSPH)
   // working arrays
@@ -90,7 +90,7 @@ void launch_rescale(float* a, int na, float* b, int nb, uint32_t* maxbits, int* 
 void launch_fill_f4(float4* a, int n, hipStream_t st);
 void launch_fill_f64(double* a, int n, hipStream_t st);
 // Caller-layout vector array -> float4.
-void launch_to_f4(int layout, const float* a, int n, float4* out, hipStream_t st);
+void launch_to_f4(const float* a, int n, float4* out, hipStream_t st);
 // out[0] = sum of a[0..n) in a fixed order (one workgroup).
 // Fixed-order sum of n doubles into out[0]; part holds 1024 doubles.
 void launch_sum_f64(const double* a, int n, double* part, double* out, hipStream_t st);
