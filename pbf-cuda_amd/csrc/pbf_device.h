@@ -600,6 +600,14 @@ __device__ __forceinline__ void sweep_seq(const SeqTable& st, uint32_t m, uint32
   }
 }
 
+// Orders the wavefront's LDS accesses (its lanes run in lockstep and the LDS
+// serves them in issue order, so only the compiler must not move them).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Exclusive prefix sum of v over the active lanes of the wavefront; *total
 // receives the sum.  All active lanes must call it.
 __device__ __forceinline__ uint32_t wave_exclusive_sum(uint32_t v, uint32_t* total) {

@@ -13,14 +13,6 @@
 namespace pbf {
 namespace {
 
-// Orders the wavefront's LDS accesses (its lanes run in lockstep and the LDS
-// serves them in issue order, so only the compiler must not move them).
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // What the team kernel needs of a pass policy besides the lane kernels'
 // hooks (pbf_pass.h): Term, one candidate's contribution; term(), which
 // forms it; fold(), which adds it to a running sum with the operations

@@ -10,9 +10,15 @@
 //   k_radix_scan_rows one workgroup per digit: exclusive scan of its row
 //   k_radix_scatter   LDS-staged stable ranking of the tile, then coalesced
 //                     scatter of runs of equal digits
-// Stability: inside a tile, equal digits are ranked in index order (items
-// processed in index order, wave64 ballot matching inside an item, per-wave
-// prefix across the 4 waves); across tiles, by the row scan.
+// Stability: inside a tile, equal digits are ranked in index order (each
+// wavefront takes a quarter of the tile in order, wave64 ballot matching
+// inside 64 items, a prefix across the 4 wavefronts); across tiles, by the row
+// scan.
+// Bound: latency at 1M pairs (a pass moves 20 MB, 4 us at the copy rate, in
+// three launches), the scatter's LDS and ballots at 4M.  Quarters instead of
+// every wavefront ranking every fourth 64 items, two barriers for each, and
+// scans in registers: scatter pass 13.6 -> 11.1 us at 1M, 35.3 -> 28.6 at 4M;
+// spread 1M step 1036 -> 1024 us, dense 2115 -> 2094.
 #include "pbf_device.h"
 #include "pbf_launch.h"
 
@@ -42,21 +48,24 @@ __device__ __forceinline__ uint64_t match_digit(uint32_t d, int bits) {
   return m;
 }
 
-// Exclusive scan over the 256 threads of the workgroup; *total gets the sum.
+// Exclusive scan over the 256 threads of the workgroup, each wavefront's in
+// registers; *total gets the sum.  s: kWaves words that no earlier reader
+// still needs.
 __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s, uint32_t* total) {
-  const int tid = threadIdx.x;
-  s[tid] = v;
+  uint32_t sum;
+  uint32_t ex = wave_exclusive_sum(v, &sum);
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) s[w] = sum;
   __syncthreads();
-  for (int off = 1; off < kSortBlock; off <<= 1) {
-    const uint32_t t = tid >= off ? s[tid - off] : 0u;
-    __syncthreads();
-    s[tid] += t;
-    __syncthreads();
+  uint32_t all = 0u;
+#pragma unroll
+  for (int k = 0; k < kWaves; ++k) {
+    const uint32_t c = s[k];
+    if (k < w) ex += c;
+    all += c;
   }
-  const uint32_t incl = s[tid];
-  *total = s[kSortBlock - 1];
-  __syncthreads();
-  return incl - v;
+  *total = all;
+  return ex;
 }
 
 __global__ __launch_bounds__(kSortBlock) void k_radix_hist(const uint32_t* __restrict__ keys, int n,
@@ -85,14 +94,15 @@ __global__ __launch_bounds__(kSortBlock) void k_radix_hist(const uint32_t* __res
 __global__ __launch_bounds__(kSortBlock) void k_radix_scan_rows(uint32_t* __restrict__ hist,
                                                                 int num_tiles,
                                                                 uint32_t* __restrict__ totals) {
-  __shared__ uint32_t s[kSortBlock];
+  __shared__ uint32_t s[2][kWaves];
   uint32_t* row = hist + (size_t)blockIdx.x * num_tiles;
   uint32_t running = 0u;
   for (int c0 = 0; c0 < num_tiles; c0 += kSortBlock) {
     const int t = c0 + (int)threadIdx.x;
     const uint32_t v = t < num_tiles ? row[t] : 0u;
     uint32_t tot;
-    const uint32_t ex = block_exclusive_scan(v, s, &tot);
+    // two areas in turn: the second barrier since frees the other one
+    const uint32_t ex = block_exclusive_scan(v, s[(c0 / kSortBlock) & 1], &tot);
     if (t < num_tiles) row[t] = running + ex;
     running += tot;
   }
@@ -105,11 +115,10 @@ __global__ __launch_bounds__(kSortBlock) void k_radix_scatter(
     const uint32_t* __restrict__ hist, const uint32_t* __restrict__ totals) {
   __shared__ uint32_t s_key[kSortTile];
   __shared__ uint32_t s_val[kSortTile];
-  __shared__ uint32_t wcnt[2][kWaves][kRadix];
-  __shared__ uint32_t dtot[kRadix];
+  __shared__ uint32_t wcnt[kWaves][kRadix];
   __shared__ uint32_t dstart[kRadix];
   __shared__ uint32_t gbase[kRadix];
-  __shared__ uint32_t scan_tmp[kRadix];
+  __shared__ uint32_t scan_tmp[2][kWaves];
 
   const int tid = threadIdx.x;
   const int w = tid >> 6;
@@ -117,68 +126,60 @@ __global__ __launch_bounds__(kSortBlock) void k_radix_scatter(
   const int base = tile * kSortTile;
   const uint32_t mask = (1u << bits) - 1u;
   const uint64_t lt = lanemask_lt();
-
-  {
-    // global start of each digit for this tile: all smaller digits of every
-    // tile + this digit in earlier tiles
-    uint32_t tot;
-    const uint32_t ex = block_exclusive_scan(totals[tid], scan_tmp, &tot);
-    gbase[tid] = ex + hist[(size_t)tid * num_tiles + tile];
-  }
-  dtot[tid] = 0u;
-  for (int ww = 0; ww < kWaves; ++ww) {
-    wcnt[0][ww][tid] = 0u;
-    wcnt[1][ww][tid] = 0u;
-  }
+  // wavefront w takes the tile's items [w, w + 1) * 64 * kSortItems in order
+  const int first = base + w * 64 * kSortItems + (tid & 63);
 
   uint32_t key[kSortItems], val[kSortItems], rank[kSortItems];
 #pragma unroll
   for (int k = 0; k < kSortItems; ++k) {
-    const int i = base + k * kSortBlock + tid;
+    const int i = first + k * 64;
     key[k] = i < n ? kin[i] : 0u;
     val[k] = i < n ? vin[i] : 0u;
   }
+  {
+    // global start of each digit for this tile: all smaller digits of every
+    // tile + this digit in earlier tiles
+    uint32_t tot;
+    const uint32_t ex = block_exclusive_scan(totals[tid], scan_tmp[0], &tot);
+    gbase[tid] = ex + hist[(size_t)tid * num_tiles + tile];
+  }
+#pragma unroll
+  for (int ww = 0; ww < kWaves; ++ww) wcnt[ww][tid] = 0u;
   __syncthreads();
 
+  // ranks within the wavefront's items: its own counters, so nothing waits
+  // for the other wavefronts
 #pragma unroll
   for (int k = 0; k < kSortItems; ++k) {
-    const int i = base + k * kSortBlock + tid;
-    const bool valid = i < n;
+    const bool valid = first + k * 64 < n;
     const uint32_t d = (key[k] >> shift) & mask;
     const uint64_t peers = match_digit(d, bits) & __ballot(valid);
     const uint32_t below = (uint32_t)__popcll(peers & lt);
-    const int par = k & 1;
-    if (valid && below == 0u) wcnt[par][w][d] = (uint32_t)__popcll(peers);
-    __syncthreads();
-    {
-      // thread tid owns digit tid: prefix over the waves of this item on top
-      // of the counts of earlier items; clears the other parity's table for
-      // the next item
-      uint32_t run = dtot[tid];
-      for (int ww = 0; ww < kWaves; ++ww) {
-        const uint32_t cc = wcnt[par][ww][tid];
-        wcnt[par][ww][tid] = run;
-        run += cc;
-        wcnt[par ^ 1][ww][tid] = 0u;
-      }
-      dtot[tid] = run;
-    }
-    __syncthreads();
-    rank[k] = valid ? wcnt[par][w][d] + below : 0u;
+    const uint32_t before = wcnt[w][d];
+    wave_lds_sync();
+    if (valid && below == 0u) wcnt[w][d] = before + (uint32_t)__popcll(peers);
+    wave_lds_sync();
+    rank[k] = before + below;
   }
-
   __syncthreads();
   {
+    // thread tid owns digit tid: prefix over the wavefronts, then over the digits
+    uint32_t run = 0u;
+#pragma unroll
+    for (int ww = 0; ww < kWaves; ++ww) {
+      const uint32_t cc = wcnt[ww][tid];
+      wcnt[ww][tid] = run;
+      run += cc;
+    }
     uint32_t tot;
-    dstart[tid] = block_exclusive_scan(dtot[tid], scan_tmp, &tot);
+    dstart[tid] = block_exclusive_scan(run, scan_tmp[1], &tot);
   }
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < kSortItems; ++k) {
-    const int i = base + k * kSortBlock + tid;
-    if (i < n) {
+    if (first + k * 64 < n) {
       const uint32_t d = (key[k] >> shift) & mask;
-      const uint32_t p = dstart[d] + rank[k];
+      const uint32_t p = dstart[d] + wcnt[w][d] + rank[k];
       if (p < (uint32_t)kSortTile) {
         s_key[p] = key[k];
         s_val[p] = val[k];
