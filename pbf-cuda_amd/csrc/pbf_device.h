@@ -129,11 +129,19 @@ constexpr uint32_t kChunk = 64;
 // A target is heavy when it has more than kLightMax candidates, or more than
 // the threshold the previous neighbour pass chose: the smallest level L of
 // heavy_level() such that at most n / kLevelShare targets had L < m <=
-// kLightMax (else kLightMax).  A light wavefront lasts as long as its longest
+// kLightMax, or, among the lowest kFewLevels, at most kFewHeavy (else
+// kLightMax).  A light wavefront lasts as long as its longest
 // lane, so in sparse water the few long lanes set the light kernel's tail and
 // are better spread over the chunk kernel (threshold 64); in dense water long
 // lanes are common, balance each other within the wavefronts, and spreading
-// them would only lengthen the chunk lists (threshold up to kLightMax).
+// them would only lengthen the chunk lists (threshold up to kLightMax).  While
+// their chunks leave the chip idle even that costs less than waiting for them,
+// if no light target is left with more than about one chunk (kFewLevels):
+// collapsing dams after 20 / 50 frames, 92K particles 797 / 833 -> 632 / 669 us a
+// step, 128K 823 / 861 -> 656 / 697, 256K 858 / 829 -> 777 / 761, fresh lattices
+// and 1M unchanged.  kFewHeavy = 65536 put a fresh 92K lattice's targets
+// on the lists (397 -> 570 us), 16384 left 256K at 841 / 785; with every level
+// a dense dam of 130,000 takes 592 us instead of 587.
 // Which targets are heavy changes no result (the canonical order above),
 // only the timing.
 constexpr uint32_t kLightMax = 256;
@@ -142,6 +150,8 @@ __host__ __device__ constexpr uint32_t heavy_level(int k) {  // 64, 80, .., 128,
   return k < 4 ? 64u + 16u * (uint32_t)k : 128u + 32u * (uint32_t)(k - 4);
 }
 constexpr uint32_t kLevelShare = 25;
+constexpr int kFewLevels = 3;  // up to 96 candidates
+constexpr uint32_t kFewHeavy = 32768;
 // The per-level counts travel packed, three 21-bit fields to a 64-bit word
 // (exact while a statistics slot counts fewer than 2^21 targets per level,
 // i.e. below 2^27 targets; beyond that a count may spill into the next field

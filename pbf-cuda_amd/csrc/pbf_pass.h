@@ -465,7 +465,9 @@ __global__ __launch_bounds__(kBlock) void k_combine(typename P::Args a, int n, S
       uint32_t thr = kLightMax;
 #pragma unroll
       for (int k = kLevels - 1; k >= 0; --k)
-        if (cnt[k] * kLevelShare <= (unsigned long long)n) thr = heavy_level(k);
+        if (cnt[k] * kLevelShare <= (unsigned long long)n ||
+            (k < kFewLevels && cnt[k] <= kFewHeavy))
+          thr = heavy_level(k);
       hl.counters[kThresholdWord] = thr;
     }
   }
