@@ -130,7 +130,7 @@ def traced_predict_us():
         text = open(STEP_FILE).read()
     except OSError:
         return None
-    m = re.search(r"\| `k_predict_key<4, OneScene>` \| [0-9.]+ \| ([0-9.]+) \|", text)
+    m = re.search(r"\| `k_predict_key<4, OneScene[^`]*` \| [0-9.]+ \| ([0-9.]+) \|", text)
     return float(m.group(1)) if m else None
 
 
@@ -527,7 +527,7 @@ def _short_kernel(name):
 def summarize(folder, warmup, steps, windows, n=1048576):
     """Per-kernel figures of the timed frames from a rocprofv3 output folder
     of this command (no GPU work).  Finds the single-dam steps by their
-    predict kernel (k_predict_key<4, OneScene> over n particles): the eager
+    predict kernel (k_predict_key<4, OneScene, ..> over n particles): the eager
     run's `warmup` steps, the autotuner's steps, its `steps` timed steps, then
     the graph run's `warmup` + steps * (1 + windows) steps.  Prints, for the
     eager and the graph run's headline window, each kernel's launches per
@@ -553,7 +553,7 @@ def summarize(folder, warmup, steps, windows, n=1048576):
                 c = disp[d][4]
                 c[r["Counter_Name"]] = c.get(r["Counter_Name"], 0.0) + float(r["Counter_Value"])
     order = sorted(disp)
-    pred = [k for k in order if "k_predict_key<4, pbf::OneScene>" in disp[k][0]
+    pred = [k for k in order if "k_predict_key<4, pbf::OneScene" in disp[k][0]
             and disp[k][1] >= n and disp[k][1] < n + 256]
     tuned = len(pred) - 2 * warmup - steps * (2 + windows)
     if tuned < 0:
@@ -586,7 +586,7 @@ def summarize(folder, warmup, steps, windows, n=1048576):
                 row += "; per launch " + ", ".join(
                     f"{c} {sum(d[4].get(c, 0.0) for d in ds) / len(ds):.6g}" for c in cnames)
             lines.append(row)
-        lam = [nm for nm in per if "<LambdaPass, OneScene>" in nm]
+        lam = [nm for nm in per if "<LambdaPass, OneScene" in nm]
         if lam:
             launches = len(per[[x for x in lam if x.startswith("k_light")][0]])
             us = sum(d[3] - d[2] for x in lam for d in per[x]) / launches / 1e3
