@@ -52,9 +52,9 @@ void launch_cell_starts(uint32_t* cnt, long long cells, uint32_t* tile_sum, uint
 // Up to how many particles a grid is built by counting (predict / key_only with
 // cnt, then launch_place_ranked) instead of the radix sort (cnt null).  Steps
 // under graph replay, radix -> counted, fresh lattice / dam after 20 frames /
-// after 50: 2K particles 182 / 146 / 147 -> 138 / 106 / 105 us, 128K 477 / 906 /
-// 911 -> 411 / 861 / 875, 512K 886 / 1343 / 1126 -> 825 / 1329 / 1104, 1M 1459 /
-// 2778 / 1860 -> 1387 / 2824 / 1865: there the step's atomics, one per run of
+// after 50: 2K particles 172 / 139 / 138 -> 143 / 101 / 103 us, 128K 447 / 688 /
+// 725 -> 392 / 656 / 696, 512K 853 / 1207 / 998 -> 800 / 1206 / 993, 1M 1338 /
+// 2245 / 1527 -> 1282 / 2293 / 1552: there the step's atomics, one per run of
 // equal keys in the previous frame's order, cost what the sort did.  A density
 // error on a finished frame's order has longer runs: 1M 329 / 412 / 262 -> 259 /
 // 396 / 244 (60 frames), 2M 489 / 666 / 523 -> 406 / 636 / 515.

@@ -503,12 +503,12 @@ int grid_for_items(long long items, int max_blocks) {
 
 // Lanes per target for n particles: 0 = the light, chunk and combine kernels.
 // Steps under graph replay, microseconds, fresh lattice / collapsing dam (20
-// frames) / spread dam (50 frames): 16K particles 235 / 189 / 201 with 16
-// lanes, 225 / 217 / 227 with 8, 386 / 719 / 710 with the lane kernels; 32K
-// 326 / 317 / 220, 266 / 357 / 246 and 425 / 766 / 793; 80K with 8 lanes 413 /
-// 520 / 482, 96K 495 / 542 / 601 against 469 / 836 / 935 with the lane kernels,
-// which from there on have wavefronts enough to win where every target has
-// much the same number of candidates.
+// frames) / spread dam (50 frames): 16K particles 195 / 164 / 162 with 16
+// lanes, 184 / 195 / 187 with 8, 400 / 584 / 594 with the lane kernels; 32K
+// 214 / 313 / 225 with 8 lanes, 386 / 598 / 631 with the lane kernels; 92K 422 /
+// 446 / 424 against 398 / 611 / 671: from there on the lane kernels have
+// wavefronts enough to win where every target has much the same number of
+// candidates.
 // A fixed heavy threshold asks for the chunk kernels, so it keeps the lane
 // kernels at every size.  Every choice sums in the canonical order.
 constexpr int kTeam16Max = 20480;
@@ -527,9 +527,9 @@ inline int team_blocks(int n, int lanes) {
 // chunk kernels and every load the light kernels: 1M dense step 2264 -> 2150 us,
 // 4M sweeping-wall frame 15.65 -> 14.48 ms, 64 scenes 8.69 -> 8.25 ms.  Smaller
 // passes wait on latency, and the hits' reloads no longer find the lines that
-// screening positions brought: 128K 393 / 824 / 863 -> 409 / 846 / 894 us (fresh
-// lattice / dam after 20 and 50 frames), 512K 785 / 1216 / 1040 -> 805 / 1189 /
-// 1058.
+// screening positions brought.  Fresh lattice / dam after 20 and 50 frames,
+// positions -> coordinates: 128K 392 / 653 / 694 -> 399 / 666 / 708 us, 512K 794 /
+// 1202 / 991 -> 809 / 1171 / 1001, 1M 1349 / 2370 / 1578 -> 1338 / 2248 / 1532.
 constexpr int kCoarseMin = (1 << 19) + 1;
 inline bool coarse_screen(int n, const Shapes& sh) {
   return n >= kCoarseMin && team_lanes(n, sh) == 0;
