@@ -52,7 +52,7 @@ struct BwdFrame {
   uint32_t* qc;           // packed query cells of the positions of the current pass
   float4 *xr, *sdb;       // lambda-pass inputs: (x, dL/drho), (S, dL/dD)
   float* grho_x;          // dL/drho of the last lambda pass, from XSPH
-  double* r0;             // per-slot dL/dpho0 accumulators
+  double* r0;             // dL/dpho0 accumulators, of which only the sum counts
   const BwdQuery* q;      // gather mode's arrays; null: scatter mode
   const int* escale;      // rescaled adjoints: true = stored x 2^*escale (r0 gets true
                           // values); null: no rescaling
