@@ -109,7 +109,7 @@ __global__ __launch_bounds__(kTeamBlock) void k_team(typename P::Args a, int n, 
   using Term = typename TT::Term;
   using Acc = typename P::Acc;
   using Target = typename P::Target;
-    // queue the candidate itself where the term needs nothing else and the
+  // queue the candidate itself where the term needs nothing else and the
   // queue is small (16 bytes an entry cost occupancy at G = 8: 64K particles
   // ran 3-5% slower than with byte offsets reloaded), else its byte offset
   constexpr bool kVecQ = TT::kNbIsScreen && G >= 16;
