@@ -1759,10 +1759,12 @@ int pbf_tape_backward(pbf_solver* s, pbf_tape* t, const float* gpos, const float
   rec.rho = rho.data();
   int cur = 0;
   // Neighbour passes of the adjoint kernels: after a recompute they follow
-  // its passes 0 .. 2 niter - 1 (it leaves out XSPH); a stored tape numbers
-  // them on from the forward run's last pass (any full step leaves the odd
-  // parity's counters cleared).
-  int pass = 2 * NI + 1;
+  // its passes 0 .. 2 niter - 1 (it leaves out XSPH).  A stored tape's begin
+  // at 0, with the work lists' counters of both parities cleared here: what
+  // ran last on the solver may have been another backward pass, whose last
+  // pass leaves its own parity's counts.
+  int pass = 0;
+  if (t->store) pbf::launch_fill_u32(s->counters, pbf::kThresholdWord, 0u, st);
   for (int f = t->nframes - 1; f >= 0; --f) {
     // frame f under its own box
     s->ulim = t->ul[(size_t)f];

@@ -668,6 +668,7 @@ __host__ __device__ __forceinline__ int rec_counter(int parity) {
 __host__ __device__ __forceinline__ int item_counter(int parity) {
   return (2 * parity + 1) * kCounterLine;
 }
+static_assert(3 * kCounterLine < kThresholdWord, "words below the threshold: the counters");
 
 // x^n for the s_corr exponent: repeated multiplication for small integer n
 // (the reference default n=4), powf otherwise.
