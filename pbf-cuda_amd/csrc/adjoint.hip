@@ -493,9 +493,11 @@ struct BwdLambdaPass {
     const float3 d = make_float3(dx, dy, dz);
     const Members mb = members<kGather>(t.cell, t.c, nb.x, nb.c, c);
     if (!(mb.own || mb.other)) return;  // no term: nothing of j may enter (0 * inf)
-    // density: the coefficient of d in both terms
-    float k = ((mb.own ? t.x.w : 0.0f) + (mb.other ? nb.x.w : 0.0f)) *
-              poly6_slope(fmaxf(c.h2 - r2, 0.0f), c);
+    // density: the coefficient of d in both terms (from h on there is no term,
+    // whatever the adjoint: 0 * inf)
+    float k = r2 < c.h2 ? ((mb.own ? t.x.w : 0.0f) + (mb.other ? nb.x.w : 0.0f)) *
+                              poly6_slope(c.h2 - r2, c)
+                        : 0.0f;
     float phi = 0.0f;
     float3 V = make_float3(0.0f, 0.0f, 0.0f);
     const Root root = root_pair(r2);
