@@ -327,7 +327,11 @@ int pbf_autotune(pbf_solver* s, const float* pos, const float* vel, const uint32
  *   not modified); the final state is pbf_tape_state(t, nframes).  With a
  *   sweep, frame k runs in the box pbf_sweep_box(sweep, first_frame + k)
  *   (as pbf_run_frames; the solver keeps the last box); the backward pass
- *   differentiates each frame in its own box.
+ *   differentiates each frame in its own box.  `s` may be another solver than
+ *   the tape's, here and in pbf_tape_backward, if its device, layout and niter
+ *   are the same, its capacity holds the tape's particles and, for a stored
+ *   tape, the box needs no more cells than the max_cells of the solver the
+ *   tape was made for (else PBF_ERR_STATE or PBF_ERR_CAPACITY).
  * pbf_tape_state: device pointers of checkpoint `frame` (0 = the inputs,
  *   nframes = the final state; caller layout, sorted as the frames left it).
  * pbf_tape_read: copies checkpoint `frame` into caller arrays (any may be

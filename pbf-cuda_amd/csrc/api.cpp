@@ -158,6 +158,7 @@ struct pbf_solver {
 struct pbf_tape {
   int device = 0;
   int n = 0, nframes = 0, niter = 0, layout = PBF_LAYOUT_FLOAT4;
+  long long max_cells = 0;           // a stored tape's cell-start tables hold this many
   bool forward_done = false;
   void* arena = nullptr;
   std::vector<float*> cpos, cvel;    // per checkpoint 0..nframes (caller layout)
@@ -1415,6 +1416,7 @@ int pbf_tape_create_ex(pbf_solver* s, int n, int nframes, int flags, pbf_tape** 
   t->nframes = nframes;
   t->niter = s->prm.niter;
   t->layout = s->layout;
+  t->max_cells = s->max_cells;
   t->store = (flags & PBF_TAPE_STORE) != 0;
   t->adjoint_flag = flags & (PBF_TAPE_GATHER | PBF_TAPE_SCATTER);
   t->rescale = (flags & PBF_TAPE_RESCALE) != 0;
@@ -1586,6 +1588,9 @@ int pbf_tape_forward(pbf_solver* s, pbf_tape* t, const float* pos, const float* 
   if (t->device != s->device || t->layout != s->layout || t->niter != s->prm.niter)
     return fail(s, PBF_ERR_STATE, "tape made for another solver state (device, layout or niter)");
   int rc;
+  // the tape may have been made for another solver: its particles must fit this
+  // one's scratch and, below, this one's grid a stored tape's tables
+  if ((rc = check_step_count(s, t->n))) return rc;
   if ((rc = check_vec_ptr(s, pos, "pos")) || (rc = check_vec_ptr(s, vel, "vel"))) return rc;
   if (!iid) return fail(s, PBF_ERR_INVALID_ARGUMENT, "iid is NULL");
   DeviceGuard g(s->device);
@@ -1618,13 +1623,16 @@ int pbf_tape_forward(pbf_solver* s, pbf_tape* t, const float* pos, const float* 
                          t->ciid[fb + 1],  t->n,            t->cpos[fb], t->cvel[fb],
                          t->ciid[fb]};
     if (!t->store) {
-      if ((rc = check_step_count(s, t->n)) || (rc = run_step(s, arr, stream))) return rc;
+      if ((rc = run_step(s, arr, stream))) return rc;
       continue;
     }
     // stored tape: the step keeps its iterations, the grid, the sort and the
     // pre-XSPH state the adjoint reads in frame f's arrays
     pbf::StepConsts c;
     if ((rc = step_consts(s, c))) return rc;
+    if (c.cells > t->max_cells)
+      return fail(s, PBF_ERR_CAPACITY, "box needs %d cells, the stored tape was made for %lld",
+                  c.cells, t->max_cells);
     const size_t q0 = fb * (size_t)t->niter;
     Record rec;
     rec.cs = t->f_cs[fb];
@@ -1659,6 +1667,9 @@ int pbf_tape_backward(pbf_solver* s, pbf_tape* t, const float* gpos, const float
   if (!t) return fail(s, PBF_ERR_INVALID_ARGUMENT, "tape is NULL");
   if (!t->forward_done) return fail(s, PBF_ERR_STATE, "pbf_tape_forward has not run on this tape");
   if (t->device != s->device) return fail(s, PBF_ERR_STATE, "tape made on another device");
+  if (s->nscenes) return fail(s, PBF_ERR_STATE, "tapes are for single-scene solvers");
+  if (t->n > s->capacity)
+    return fail(s, PBF_ERR_CAPACITY, "the tape's n = %d exceeds capacity %d", t->n, s->capacity);
   if (std::memcmp(&t->prm, &s->prm, sizeof(pbf_params)) != 0 || t->layout != s->layout)
     return fail(s, PBF_ERR_STATE, "parameters changed since the forward run");
   int rc;
