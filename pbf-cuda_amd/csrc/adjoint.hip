@@ -784,14 +784,17 @@ __global__ __launch_bounds__(kBlock) void k_bwd_fold(int n, const float4* __rest
 }
 
 // Per-frame rescaling of the adjoint state (tapes with PBF_TAPE_RESCALE):
-// the largest finite |value| of two arrays, as float bits (all values are
+// the largest finite |value| of two arrays of layout L (4: each fourth value is
+// padding, which counts for nothing), as float bits (all values are
 // non-negative, so the unsigned order of the bits is the float order) ...
+template <int L>
 __global__ __launch_bounds__(kBlock) void k_absmax(const float* __restrict__ a, int na,
                                                    const float* __restrict__ b, int nb,
                                                    uint32_t* __restrict__ out) {
   uint32_t m = 0u;
   const int stride = gridDim.x * kBlock;
   for (int k = blockIdx.x * kBlock + threadIdx.x; k < na + nb; k += stride) {
+    if (L == 4 && (k & 3) == 3) continue;
     const float v = fabsf(k < na ? a[k] : b[k - na]);
     const uint32_t bits = __float_as_uint(v);
     m = (v <= 3.4028235e38f && bits > m) ? bits : m;  // NaN and inf are left out
@@ -1025,12 +1028,16 @@ void launch_bwd_predict(int layout, const BwdFrame& f, const uint32_t* sval, int
     k_bwd_predict<4><<<blocks_for(n), kBlock, 0, st>>>(n, c, sval, f.gx, f.gx0, gpos, gvel);
 }
 
-void launch_rescale(float* a, int na, float* b, int nb, uint32_t* maxbits, int* escale,
+void launch_rescale(int layout, float* a, float* b, int n, uint32_t* maxbits, int* escale,
                     hipStream_t st) {
   k_fill_u32_one<<<1, 64, 0, st>>>(maxbits);
-  const int blocks = fill_blocks(na + nb);
-  k_absmax<<<blocks, kBlock, 0, st>>>(a, na, b, nb, maxbits);
-  k_rescale<<<blocks, kBlock, 0, st>>>(a, na, b, nb, maxbits, escale);
+  const int m = n * layout;
+  const int blocks = fill_blocks(m + m);
+  if (layout == 4)
+    k_absmax<4><<<blocks, kBlock, 0, st>>>(a, m, b, m, maxbits);
+  else
+    k_absmax<3><<<blocks, kBlock, 0, st>>>(a, m, b, m, maxbits);
+  k_rescale<<<blocks, kBlock, 0, st>>>(a, m, b, m, maxbits, escale);
 }
 
 void launch_fill_f4(float4* a, int n, hipStream_t st) {

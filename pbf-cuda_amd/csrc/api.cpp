@@ -1707,7 +1707,7 @@ int pbf_tape_backward(pbf_solver* s, pbf_tape* t, const float* gpos, const float
   pbf::launch_fill_f64(t->r0, n, st);
   if (t->rescale) {
     pbf::launch_fill_u32(reinterpret_cast<uint32_t*>(t->escale), 1, 0u, st);
-    pbf::launch_rescale(t->gp[0], n * L, t->gv[0], n * L, t->maxbits, t->escale, st);
+    pbf::launch_rescale(L, t->gp[0], t->gv[0], n, t->maxbits, t->escale, st);
   }
   // Adjoint mode: gather (each pass over a grid of its own positions, no
   // atomics) from kGatherMinParticles particles or on request, when every
@@ -1849,7 +1849,7 @@ int pbf_tape_backward(pbf_solver* s, pbf_tape* t, const float* gpos, const float
     float* op = f == 0 ? gpos0 : t->gp[cur ^ 1];
     float* ov = f == 0 ? gvel0 : t->gv[cur ^ 1];
     pbf::launch_bwd_predict(L, bf, sval, n, c, op, ov, st);
-    if (t->rescale && f > 0) pbf::launch_rescale(op, n * L, ov, n * L, t->maxbits, t->escale, st);
+    if (t->rescale && f > 0) pbf::launch_rescale(L, op, ov, n, t->maxbits, t->escale, st);
     gp_in = op;
     gv_in = ov;
     cur ^= 1;

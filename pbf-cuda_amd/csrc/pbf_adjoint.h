@@ -83,10 +83,11 @@ void launch_bwd_iteration(const BwdFrame& f, const BwdIter& it, int last, int n,
 void launch_bwd_predict(int layout, const BwdFrame& f, const uint32_t* sval, int n,
                         const StepConsts& c, float* gpos, float* gvel, hipStream_t st);
 
-// Rescales the adjoint arrays a (na floats) and b (nb floats) by a power of
-// two so that their largest finite |value| lies in [1, 2), and subtracts the
-// exponent applied from *escale (maxbits: one device word of scratch).
-void launch_rescale(float* a, int na, float* b, int nb, uint32_t* maxbits, int* escale,
+// Rescales the adjoint arrays a and b (n vectors of the layout each) by a power
+// of two so that their largest finite |value| (padding left out) lies in
+// [1, 2), and subtracts the exponent applied from *escale (maxbits: one device
+// word of scratch).
+void launch_rescale(int layout, float* a, float* b, int n, uint32_t* maxbits, int* escale,
                     hipStream_t st);
 void launch_fill_f4(float4* a, int n, hipStream_t st);
 void launch_fill_f64(double* a, int n, hipStream_t st);
