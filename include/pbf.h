@@ -173,9 +173,10 @@ int pbf_density_error(pbf_solver* s, const float* pos, int n, void* stream,
  * fluids/Logger.cpp:17-82, fluids/Simulator.cpp:44-79, without device-wide
  * syncs).  enable != 0 starts recording; records are resolved by
  * pbf_get_timing, which synchronises the recorded events. */
-#define PBF_PHASE_PREDICT 0 /* predict + cell key */
-#define PBF_PHASE_SORT 1    /* radix sort of (key, index) */
-#define PBF_PHASE_GRID 2    /* cell clear + permute + cell ranges */
+#define PBF_PHASE_PREDICT 0 /* predict + cell key (up to 2^19 particles: + counts per cell) */
+#define PBF_PHASE_SORT 1    /* radix sort of (key, index); up to 2^19 particles: cell ranges from
+                               the counts + list of the particles by cell */
+#define PBF_PHASE_GRID 2    /* permute + cell ranges; up to 2^19 particles: ranking + permute */
 #define PBF_PHASE_LAMBDA 3  /* one lambda launch */
 #define PBF_PHASE_DELTA 4   /* one delta-p launch */
 #define PBF_PHASE_VEL 5     /* velocity update: fused into the last delta-p launch, so

@@ -503,11 +503,15 @@ void enqueue_step(pbf_solver* s, const StepArrays& a, const pbf::StepConsts& c, 
   // (Simulator.cu:200-204)
   if (counted) {
     // the work lists' records are free until the first neighbour pass
+    uint2* const list = (uint2*)s->hl.recs;
+    tb(PBF_PHASE_SORT);
+    pbf::launch_count_place(s->key0, s->val0, list, n, c.cells, s->tile_sum, cs, s->cnt, st);
+    te(PBF_PHASE_SORT);
     tb(PBF_PHASE_GRID);
     uint32_t* const key = rec ? (rec->keep_key ? rec->keep_key : s->key1) : nullptr;
     uint32_t* const val = rec ? (rec->keep_val ? rec->keep_val : s->val1) : nullptr;
-    pbf::launch_place_ranked(L, s->key0, s->val0, (uint2*)s->hl.recs, in_pos, s->xp, in_iid, n, c,
-                             s->tile_sum, cs, s->x0s, xa, coarse, s->iid_s, s->cnt, key, val, st);
+    pbf::launch_permute_ranked(L, list, cs, in_pos, s->xp, in_iid, n, c, s->x0s, xa, coarse,
+                               s->iid_s, s->cnt, key, val, st);
     te(PBF_PHASE_GRID);
     if (rec) {
       rec->skey = key;
@@ -1330,9 +1334,10 @@ int pbf_density_error(pbf_solver* s, const float* pos, int n, void* stream, doub
   pbf::launch_key_only(s->layout, pos, n, c, scn, s->xp, s->key0, s->val0, s->counters,
                        counted ? s->cnt : nullptr, st);
   if (counted) {
-    pbf::launch_place_ranked(s->layout, s->key0, s->val0, (uint2*)s->hl.recs, nullptr, s->xp,
-                             nullptr, n, c, s->tile_sum, s->cs, nullptr, s->xa, coarse, nullptr,
-                             s->cnt, nullptr, nullptr, st);
+    uint2* const list = (uint2*)s->hl.recs;
+    pbf::launch_count_place(s->key0, s->val0, list, n, c.cells, s->tile_sum, s->cs, s->cnt, st);
+    pbf::launch_permute_ranked(s->layout, list, s->cs, nullptr, s->xp, nullptr, n, c, nullptr,
+                               s->xa, coarse, nullptr, s->cnt, nullptr, nullptr, st);
   } else {
     const int which = pbf::radix_sort_pairs(s->key0, s->val0, s->key1, s->val1, n,
                                             key_bits_for(c.cells), s->hist, s->totals, st);

@@ -50,7 +50,7 @@ long long scan_tiles(long long cells);
 void launch_cell_starts(uint32_t* cnt, long long cells, uint32_t* tile_sum, uint32_t* cs,
                         hipStream_t st);
 // Up to how many particles a grid is built by counting (predict / key_only with
-// cnt, then launch_place_ranked) instead of the radix sort (cnt null).  Steps
+// cnt, launch_count_place, launch_permute_ranked) instead of the radix sort (cnt null).  Steps
 // under graph replay, radix -> counted, fresh lattice / dam after 20 frames /
 // after 50: 2K particles 172 / 139 / 138 -> 143 / 101 / 103 us, 128K 447 / 688 /
 // 725 -> 392 / 656 / 696, 512K 853 / 1207 / 998 -> 800 / 1206 / 993, 1M 1338 /
@@ -66,15 +66,13 @@ constexpr int kCountedDensityMax = 1 << 21;
 void launch_count_place(const uint32_t* key, const uint32_t* arrival, uint2* list, int n,
                         long long cells, uint32_t* tile_sum, uint32_t* cs, uint32_t* cnt,
                         hipStream_t st);
-// From the counts cnt and arrival numbers of the predict kernel: the cell-start
-// table cs and the payload in the order of the stable sort; clears cnt.  list:
-// n entries of scratch.  pos null: only xa is moved.  skey, sval (may be null)
-// receive the sorted keys and their input indices.
-void launch_place_ranked(int layout, const uint32_t* key, const uint32_t* arrival, uint2* list,
-                         const float* pos, const float4* xp, const uint32_t* iid, int n,
-                         const StepConsts& c, uint32_t* tile_sum, uint32_t* cs, float4* x0s,
-                         float4* xa, uint2* coarse, uint32_t* iid_s, uint32_t* cnt,
-                         uint32_t* skey, uint32_t* sval, hipStream_t st);
+// From that list and table: the payload in the order of the stable sort; clears
+// cnt.  pos null: only xa is moved.  skey, sval (may be null) receive the sorted
+// keys and their input indices.
+void launch_permute_ranked(int layout, const uint2* list, const uint32_t* cs, const float* pos,
+                           const float4* xp, const uint32_t* iid, int n, const StepConsts& c,
+                           float4* x0s, float4* xa, uint2* coarse, uint32_t* iid_s, uint32_t* cnt,
+                           uint32_t* skey, uint32_t* sval, hipStream_t st);
 // Where the screening coordinates of a pass of n particles go (null: it screens
 // positions); coarse below and above: the place for those of xa, or null.
 uint2* coarse_of(const HeavyLists& hl, int n, const Shapes& sh);

@@ -907,12 +907,10 @@ void launch_count_place(const uint32_t* key, const uint32_t* arrival, uint2* lis
   k_place<<<blocks_for(n), kBlock, 0, st>>>(key, arrival, n, cs, list);
 }
 
-void launch_place_ranked(int layout, const uint32_t* key, const uint32_t* arrival, uint2* list,
-                         const float* pos, const float4* xp, const uint32_t* iid, int n,
-                         const StepConsts& c, uint32_t* tile_sum, uint32_t* cs, float4* x0s,
-                         float4* xa, uint2* coarse, uint32_t* iid_s, uint32_t* cnt,
-                         uint32_t* skey, uint32_t* sval, hipStream_t st) {
-  launch_count_place(key, arrival, list, n, c.cells, tile_sum, cs, cnt, st);
+void launch_permute_ranked(int layout, const uint2* list, const uint32_t* cs, const float* pos,
+                           const float4* xp, const uint32_t* iid, int n, const StepConsts& c,
+                           float4* x0s, float4* xa, uint2* coarse, uint32_t* iid_s, uint32_t* cnt,
+                           uint32_t* skey, uint32_t* sval, hipStream_t st) {
   if (!pos)
     k_permute_ranked<0><<<blocks_for(n), kBlock, 0, st>>>(list, cs, nullptr, xp, nullptr, n, c,
                                                           nullptr, xa, coarse, nullptr, cnt, skey,
