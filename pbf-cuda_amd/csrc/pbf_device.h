@@ -858,7 +858,13 @@ __device__ __forceinline__ uint32_t count_arrival(uint32_t k, bool valid,
 // Rank of entry i among the cell's entries list[lo, hi).  A cell of up to
 // kRankEntries is read by each of its lanes, eight loads in flight; a larger
 // one (a pile: consecutive slots, so whole wavefronts rank the same cell) by
-// the wavefront together, 64 entries a load, each passed to all lanes.
+// the wavefront together, four loads of 64 entries in flight: entries that all
+// lie below or above the indexes to rank are counted at once (particles arrive
+// nearly in input order, so most do), the others passed to all lanes one by one.
+// One load at a time and every entry passed, density error of 2M particles, of
+// which 5,000 / 20,000 lie in one cell: 487 / 1145 -> 451 / 999 us, in random
+// input order 625 / 1419 -> 584 / 1211 (with the radix sort 563 / 1081 and 592 /
+// 1109); a step of 200,000 with 5,000 in one cell 984 -> 942 (sort: 963).
 constexpr uint32_t kRankEntries = 64;
 __device__ __forceinline__ uint32_t rank_in_cell(const uint2* __restrict__ list, uint32_t lo,
                                                  uint32_t hi, uint32_t i, bool valid) {
@@ -880,13 +886,34 @@ __device__ __forceinline__ uint32_t rank_in_cell(const uint2* __restrict__ list,
     const uint32_t l = (uint32_t)__builtin_amdgcn_readlane((int)lo, src);
     const uint32_t h = (uint32_t)__builtin_amdgcn_readlane((int)hi, src);
     const bool mine = big & (lo == l);
-    uint32_t r = 0u;
-    for (uint32_t s = l; s < h; s += 64u) {
-      const uint32_t at = s + (uint32_t)lane;
-      const uint32_t e = at < h ? list[at].x : ~0u;
+    // the range of the indexes to rank
+    uint32_t least = mine ? i : ~0u, most = mine ? i : 0u;
 #pragma unroll
-      for (int t = 0; t < 64; ++t)
-        r += (uint32_t)__builtin_amdgcn_readlane((int)e, t) < i ? 1u : 0u;
+    for (int d = 1; d < 64; d <<= 1) {
+      const uint32_t a = __shfl_xor(least, d), b = __shfl_xor(most, d);
+      least = a < least ? a : least;
+      most = b > most ? b : most;
+    }
+    uint32_t r = 0u;
+    for (uint32_t s = l; s < h; s += 256u) {
+      uint32_t e[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t at = s + 64u * (uint32_t)q + (uint32_t)lane;
+        e[q] = at < h ? list[at].x : ~0u;
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint64_t below = __builtin_amdgcn_ballot_w64(e[q] < least);
+        const uint64_t above = __builtin_amdgcn_ballot_w64(e[q] > most);
+        if ((below | above) == ~0ull) {
+          r += (uint32_t)__popcll(below);
+          continue;
+        }
+#pragma unroll
+        for (int t = 0; t < 64; ++t)
+          r += (uint32_t)__builtin_amdgcn_readlane((int)e[q], t) < i ? 1u : 0u;
+      }
     }
     if (mine) rank = r;
     todo &= ~__builtin_amdgcn_ballot_w64(mine);
