@@ -283,7 +283,9 @@ int pbf_get_heavy_threshold(const pbf_solver* s, int* out);
  * caller's arrays are not modified), checks that every shape produced the
  * same bits, and installs the fastest.  *best and *best_ms (optional)
  * receive it and its median step time.  Allocates and synchronises.
- * n = the particle count (the total for a batched solver).
+ * n = the particle count (the total for a batched solver).  Where a step of n
+ * particles runs no kernel that has these shapes (up to 90,112 particles, see
+ * pbf_set_heavy_threshold), the current shapes are timed and stay installed.
  */
 int pbf_autotune(pbf_solver* s, const float* pos, const float* vel, const uint32_t* iid, int n,
                  int reps, void* stream, pbf_shapes* best, double* best_ms);

@@ -1195,11 +1195,14 @@ int pbf_autotune(pbf_solver* s, const float* pos, const float* vel, const uint32
   if ((e = hipEventCreate(&e0)) != hipSuccess || (e = hipEventCreate(&e1)) != hipSuccess) {
     rc = fail_hip(s, e, "hipEventCreate");
   }
-  const int blocks[3] = {64, 128, 256};
-  const int grids[4] = {512, 1024, 2048, 4096};
+  std::vector<int> blocks{64, 128, 256}, grids{512, 1024, 2048, 4096};
+  if (!pbf::uses_shapes(n, saved)) {  // one launch whatever the shape: nothing to choose
+    blocks = {saved.light_block};
+    grids = {saved.chunk_blocks};
+  }
   bool first = true;
-  for (int bi = 0; bi < 3 && rc == PBF_OK; ++bi) {
-    for (int gi = 0; gi < 4 && rc == PBF_OK; ++gi) {
+  for (size_t bi = 0; bi < blocks.size() && rc == PBF_OK; ++bi) {
+    for (size_t gi = 0; gi < grids.size() && rc == PBF_OK; ++gi) {
       s->shapes.light_block = blocks[bi];
       s->shapes.chunk_blocks = grids[gi];
       std::vector<double> t;

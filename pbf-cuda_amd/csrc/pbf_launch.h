@@ -76,6 +76,8 @@ void launch_permute_ranked(int layout, const uint2* list, const uint32_t* cs, co
 // Where the screening coordinates of a pass of n particles go (null: it screens
 // positions); coarse below and above: the place for those of xa, or null.
 uint2* coarse_of(const HeavyLists& hl, int n, const Shapes& sh);
+// Whether a pass of n particles runs the kernels whose launch shapes sh holds.
+bool uses_shapes(int n, const Shapes& sh);
 // The payload gathers after the sort also count the particles per cell from
 // the sorted keys skey into cnt (all zero beforehand), the input of
 // launch_cell_starts.

@@ -945,6 +945,8 @@ uint2* coarse_of(const HeavyLists& hl, int n, const Shapes& sh) {
   return coarse_screen(n, sh) ? hl.coarse : nullptr;
 }
 
+bool uses_shapes(int n, const Shapes& sh) { return team_lanes(n, sh) == 0; }
+
 void launch_lambda(const float4* xa, const uint32_t* cs, int n, const StepConsts& c,
                    const Scenes& scn, float4* xl, float* rho, float4* sd, const HeavyLists& hl,
                    int pass, const Shapes& sh, hipStream_t st) {

@@ -239,7 +239,7 @@ class Simulator:
     def autotune(self, pos, vel, iid, nparticle: int, reps: int = 3, stream=None):
         """Times one step from (pos, vel, iid) per candidate launch shape on
         private copies, checks every shape gives the same bits, installs the
-        fastest.  Returns ((light_block, chunk_blocks), median ms).
+        fastest (where a step uses no shape, the current ones stay).  Returns ((light_block, chunk_blocks), median ms).
         Synchronises; the arrays are not modified."""
         n = int(nparticle)
         L = self.layout
