@@ -222,8 +222,8 @@ int pbf_step_batched(pbf_solver* s, float* pos, float* npos, float* vel, float* 
  * Graph mode (no counterpart in the reference).  With enable != 0, pbf_step
  * records its launch sequence into a HIP graph the first time it sees an
  * (arrays, n, stream) combination, and replays that graph on later calls
- * with the same combination: one graph launch per step instead of ~40
- * kernel launches.  Up to 4 graphs are kept (a tic-toc needs 2).  A graph
+ * with the same combination: one graph launch per step instead of 13
+ * to 40 kernel launches.  Up to 4 graphs are kept (a tic-toc needs 2).  A graph
  * stays valid across parameter, box and shape changes: when pbf_set_params
  * (with new values), pbf_set_lim or pbf_set_shapes changed what the
  * sequence depends on, the next step with that combination records it
@@ -267,11 +267,18 @@ int pbf_get_shapes(const pbf_solver* s, pbf_shapes* out);
  * candidate neighbours than the threshold has its 64-candidate chunks spread
  * over the chunk kernel instead of one lane.  0 (the default) = adaptive:
  * the smallest of 64, 80, 96, 112, 128, 160, 192 such that the previous
- * neighbour pass found at most 1 in 25 targets with more candidates than it
- * and at most 256, else 256; otherwise a fixed count >= 64.  Like the launch
- * shapes, it changes no result of a step, only the speed.  Steps of up to
- * 90,112 particles have no chunk kernel under the adaptive setting (a team of
- * lanes per target instead); a fixed count keeps them on the chunk kernel.
+ * neighbour pass found at most 1 in 25 targets (for 64, 80 and 96: or at most
+ * 32,768, whatever their share) with more candidates than it and at most 256,
+ * else 256; otherwise a fixed count >= 64.  Like the launch shapes, it changes
+ * no result of a step, only the speed.  Steps of up to 90,112 particles have
+ * no chunk kernel under the adaptive setting (a team of lanes per target
+ * instead); a fixed count keeps them on the chunk kernel.  That is the faster
+ * way for small scenes with a pile of some thousand particles in one cell
+ * (80,000 particles, 4,000 of them in one cell: 0.76 ms a step instead of
+ * 2.4), the slower one for most others.  Up to 90,112 particles the last bits
+ * of a tape's gradients depend on which of the two kinds of kernels ran (they
+ * add the same terms in another grouping), so a gather-mode backward pass
+ * repeats bit for bit under one setting, not across the two.
  */
 int pbf_set_heavy_threshold(pbf_solver* s, int threshold);
 int pbf_get_heavy_threshold(const pbf_solver* s, int* out);
@@ -316,8 +323,9 @@ int pbf_autotune(pbf_solver* s, const float* pos, const float* vel, const uint32
  *   PBF_ERR_INVALID_ARGUMENT).  SCATTER lets i add such a term to j with a
  *   float atomic (the summation order, and so the last bits, can vary from
  *   run to run).  Without either flag, tapes of 2^18 particles or more
- *   gather when their grids allow it and smaller tapes scatter (there the
- *   per-pass sort of the gather costs more than the atomics).
+ *   gather when their grids allow it and smaller tapes scatter (up to about
+ *   90,000 particles the gather's per-pass grids cost more than the atomics,
+ *   up to 200,000 about as much).
  *   PBF_TAPE_RESCALE: before the backward pass of each frame the adjoint
  *   state is multiplied by a power of two that brings its largest finite
  *   magnitude into [1, 2), so gradients that grow by many orders of

@@ -69,7 +69,7 @@ class Simulator {
     const pbf_shapes sh{light_block, chunk_blocks};
     check(pbf_set_shapes(s_, &sh), s_);
   }
-  // 0 = adaptive (default); results never depend on it.
+  // 0 = adaptive (default); no result of a step depends on it (pbf.h).
   void setHeavyThreshold(int threshold) { check(pbf_set_heavy_threshold(s_, threshold), s_); }
   pbf_shapes autotune(const float* pos, const float* vel, const uint32_t* iid, int n, int reps = 3,
                       void* stream = nullptr, double* best_ms = nullptr) {

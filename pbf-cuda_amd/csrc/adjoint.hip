@@ -228,7 +228,8 @@ template <bool kGather>
 struct BwdXsphPass {
   // scatter mode: workgroups in launch order, round-robin over the XCDs, so a
   // crowded cell's targets scatter from all eight XCDs, each into its own
-  // copy; gather mode: runs of workgroups
+  // copy; gather mode: runs of workgroups (the team kernel: one contiguous
+  // range per XCD in both, so there such a cell uses one copy)
   static constexpr bool kXcdRanges = kGather;
   static constexpr bool kCoarse = kGather;
   // hits reloaded per round of the sweep

@@ -28,8 +28,8 @@ struct BwdQuery {
 // Scatter mode's copies of the scattered pair sums: workgroup b adds to copy b % 8 (the XCD
 // it runs on, as workgroups are dispatched round-robin), which spreads the
 // atomic adds a crowded cell sends to one particle over eight addresses
-// (same-address atomics serialise); the next pointwise kernel adds the
-// copies.
+// (same-address atomics serialise) where its targets are spread over the XCDs
+// (the lane kernels); the next pointwise kernel adds the copies.
 constexpr int kScatterCopies = 8;
 
 // One frame's backward state.

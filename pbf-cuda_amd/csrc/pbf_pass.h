@@ -505,10 +505,17 @@ int grid_for_items(long long items, int max_blocks) {
 // Steps under graph replay, microseconds, fresh lattice / collapsing dam (20
 // frames) / spread dam (50 frames): 16K particles 195 / 164 / 162 with 16
 // lanes, 184 / 195 / 187 with 8, 400 / 584 / 594 with the lane kernels; 32K
-// 214 / 313 / 225 with 8 lanes, 386 / 598 / 631 with the lane kernels; 92K 422 /
-// 446 / 424 against 398 / 611 / 671: from there on the lane kernels have
-// wavefronts enough to win where every target has much the same number of
-// candidates.
+// 214 / 313 / 225 with 8 lanes, 386 / 598 / 631 with the lane kernels; 93K 383 /
+// 429 / 474 against 335 / 587 / 642, 130K 498 / 559 / 636 against 344 / 608 / 699.
+// Where every target has much the same number of candidates the lane kernels win
+// from about 85K on (360 against 331), in dams teams win up to 130K and beyond, by
+// less and less; nothing the host knows tells the two apart, and the line keeps a
+// lattice's loss to about a tenth.
+// Piles of one to seven thousand particles in one cell are the teams' worst case
+// (a team's item is 64 candidates of one target, of which every lane folds every
+// term): 80,000 particles, 1,000 / 2,000 / 4,000 / 6,000 of them in one cell 641 /
+// 1060 / 2411 / 4391 us a step against 552 / 610 / 761 / 953 with the lane kernels;
+// 8,000 overflow those kernels' lists, 6724 against 8388.
 // A fixed heavy threshold asks for the chunk kernels, so it keeps the lane
 // kernels at every size.  Every choice sums in the canonical order.
 constexpr int kTeam16Max = 20480;
